@@ -337,7 +337,9 @@ PROJECTIONS = [("0.6B q", 2048, 1024), ("0.6B k/v", 1024, 1024), ("0.6B o", 1024
                ("0.6B gate/up", 3072, 1024), ("0.6B down", 1024, 3072),
                ("8B q/o", 4096, 4096), ("8B k/v", 1024, 4096), ("8B gate/up", 12288, 4096),
                ("8B down", 4096, 12288)]
-GEMM_TILES = ["128x128", "64x64", "64x32", "32x64", "32x32"]
+# tokens x outputs per tile code; "b": the bf16-piece kernel
+GEMM_TILES = ["128x128", "64x64", "64x32", "32x64", "32x32", "128x256 b", "128x128 b", "64x128 b",
+              "64x64 b"]
 
 
 def gemm_sweep(torch, ikv, tokens=(65, 128, 256, 512, 1024, 2047)):
@@ -370,7 +372,7 @@ def gemm_sweep(torch, ikv, tokens=(65, 128, 256, 512, 1024, 2047)):
                         raise RuntimeError(f"tile {t} split {sk}: {rc}")
                 return f
             tile, split = ctypes.c_int(), ctypes.c_int()
-            if blib.ikv_bench_gemm_plan(n, k, m, ctypes.byref(tile), ctypes.byref(split)):
+            if blib.ikv_bench_gemm_choice(n, k, m, ctypes.byref(tile), ctypes.byref(split)):
                 raise RuntimeError("gemm plan")
             row = {"proj": name, "n_out": n, "k": k, "tokens": m,
                    "plan": f"{GEMM_TILES[tile.value]}/s{split.value}"}
@@ -383,8 +385,8 @@ def gemm_sweep(torch, ikv, tokens=(65, 128, 256, 512, 1024, 2047)):
             for t, tname in enumerate(GEMM_TILES):
                 if t == 0 and n % 128:
                     continue
-                bm, bn = (int(v) for v in tname.split("x"))
-                n_tiles = -(-m // bm) * (n // bn)
+                bm, bn = (int(v) for v in tname.split()[0].split("x"))
+                n_tiles = -(-m // bm) * -(-n // bn)
                 cands.append((t, 1, tname))
                 cands += [(t, sk, f"{tname}/s{sk}") for sk in (2, 3, 4, 5, 6, 8)
                           if k // 64 >= 4 * sk and n_tiles * sk <= 2048

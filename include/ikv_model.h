@@ -31,7 +31,10 @@ extern "C" {
  * n_out % 16 == 0, k % 1024 == 0 and 16-byte aligned w and x runs a
  * hand-written F32 MFMA kernel. Other m > 1 with n_out % 64 == 0,
  * k % 64 == 0, k < 2^22 and 16-byte aligned w and x run the tiled F32 MFMA GEMM of
- * ikv_gemm_nt_f32, with K split over several workgroups when its tiles
+ * ikv_gemm_nt_f32 or, for products large enough, the same product on bf16
+ * MFMA with every float split into three exact bf16 pieces (F32 inputs,
+ * sums and results; no farther from a 64-bit product than the F32 MFMA
+ * kernel), with K split over several workgroups when the tiles
  * would leave compute units idle: such a call needs a split-K workspace of
  * its device and stream, which the first one allocates (8 MiB + 16 KiB,
  * kept until exit; so make it outside HIP graph capture; -ENOMEM after 64
@@ -44,7 +47,7 @@ extern "C" {
 int ikv_mul_mat_f32(const float *w, const float *x, float *out, int64_t n_out, int64_t k,
                     int64_t m, const float *residual, void *stream);
 
-/* The hand-written F32 MFMA GEMM of mul_mat for prompts (the same product,
+/* The hand-written MFMA GEMM of mul_mat for prompts (the same product,
  * CPUBackend::compute_mul_mat, src/backends/cpu_backend.cpp:386-424), for
  * any m >= 1: n_out % 64 == 0, k % 64 == 0, k < 2^22, 16-byte aligned w and x (else
  * -ENOTSUP / -EINVAL, nothing launched). Deterministic (a fixed summation

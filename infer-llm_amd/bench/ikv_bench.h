@@ -46,7 +46,8 @@ int ikv_bench_timeline_read(unsigned long long *dst, size_t n_words);
 int ikv_bench_timeline_clear(void);
 
 /* ikv_gemm_nt_f32 (include/ikv_model.h) on tile shape `tile` (tokens x
- * outputs: 0 128 x 128, 1 64 x 64, 2 64 x 32, 3 32 x 64, 4 32 x 32) with K
+ * outputs: 0 128 x 128, 1 64 x 64, 2 64 x 32, 3 32 x 64, 4 32 x 32 on F32
+ * MFMA; 5 128 x 256, 6 128 x 128, 7 64 x 128, 8 64 x 64 on bf16 pieces) with K
  * split over n_split workgroups per tile (1 <= n_split <= k / 64), for the
  * benchmark's sweep of the plans that ikv_mul_mat_f32 chooses among. For
  * n_split > 1, ws holds 16 KiB of tile counters (zero before the first
@@ -56,9 +57,11 @@ int ikv_bench_gemm_nt_tile_f32(const float *w, const float *x, float *out, int64
                                int64_t k, int64_t m, const float *residual, int tile,
                                int n_split, void *ws, size_t ws_bytes, void *stream);
 
-/* The plan ikv_mul_mat_f32 takes for an n_out x k x m product: tile code
- * (as above) and K splits, written to *tile and *n_split. */
+/* The plan of the F32 MFMA kernel for an n_out x k x m product (tile code as
+ * above and K splits, written to *tile and *n_split), and the one
+ * ikv_mul_mat_f32 takes: that or a plan of the bf16-piece kernel. */
 int ikv_bench_gemm_plan(int64_t n_out, int64_t k, int64_t m, int *tile, int *n_split);
+int ikv_bench_gemm_choice(int64_t n_out, int64_t k, int64_t m, int *tile, int *n_split);
 
 #ifdef __cplusplus
 }

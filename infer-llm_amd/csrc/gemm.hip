@@ -44,9 +44,11 @@
 //     itself on the tile's counter; the workgroup that counts last adds the
 //     partials in split order (0, 1, ..., its own from registers), writes
 //     the tile and sets the counter back to 0.
-//   * Tile shape and split (gemm_plan) come from a cost model fitted to a
-//     sweep of the Qwen3 projections on MI355X: rounds of tiles over the
-//     256 CUs times a measured time per tile of each shape.
+//   * Kernel, tile shape and split (gemm_plan) come from a cost model fitted
+//     to a sweep of the Qwen3 projections on MI355X: rounds of tiles over the
+//     256 CUs times a measured time per tile of each shape. Products with
+//     enough tiles to fill the chip go to gemm_bf16x3.hip; this kernel keeps
+//     the smaller ones, where its 32- and 64-wide tiles reach more CUs.
 //   * Results are deterministic (fixed order per output for a given shape;
 //     the split depends only on n_out, k and m).
 #include "coherent.hpp"
@@ -435,6 +437,26 @@ struct TileShape {
 constexpr TileShape kTiles[] = {{128, 128, 12.5f}, {64, 64, 3.9f}, {64, 32, 2.0f},
                                 {32, 64, 2.1f},    {32, 32, 1.0f}};
 constexpr int kNumTiles = 5;
+// The bf16-piece kernel's shapes (gemm_bf16x3.hip). A launch of T tiles split
+// S ways puts W = ceil(T * S / 256) workgroups on a CU, up to `res` of them at
+// once: us = fixed + steps / S * (W / res * us[res - 1] + us[W % res - 1]) (+
+// split + per_split * (S - 1) for S > 1), us[q - 1] the time of a 64-column
+// step of q workgroups on a CU. Fitted (non-negative least squares, 5-8% rms)
+// to 12 projection shapes (n_out 256-12288, k 768-12288) at ten token counts
+// from 72 to 4096, every split; the F32 model's units are 0.24 us there, plus
+// 4.2 us. Over that sweep the plan is on average 0.7% slower than the best
+// choice and 1.18 times as fast as the F32 kernel alone.
+struct Bf16x3Shape {
+  int bt, bw, groups, res;  // tokens, weight rows, K groups, workgroups per CU
+  double fixed, us[3], split, per_split;
+};
+constexpr Bf16x3Shape kBf16x3[] = {{128, 256, 1, 1, 9.3, {3.0, 0, 0}, 3.2, 8.2},
+                                   {128, 128, 1, 2, 5.7, {1.74, 4.11, 0}, 2.7, 4.1},
+                                   {64, 128, 1, 3, 4.1, {1.2, 2.47, 4.18}, 2.0, 2.2},
+                                   {64, 64, 2, 3, 4.6, {0.73, 1.38, 2.29}, 1.3, 2.2}};
+constexpr int kNumBf16x3 = 4;
+constexpr double kUnitUs = 0.24, kFixedUs = 4.2;
+constexpr double kBf16x3Margin = 0.95;  // taken when it promises 5% over the F32 kernel
 constexpr double kFillSteps = 2.0;
 constexpr int kMinSplitSteps = 4;   // steps of BK columns per split, at least
 constexpr int kMaxSplit = 8;
@@ -448,11 +470,21 @@ int64_t tile_count(int tile, int n, int m) {
   return int64_t((m + kTiles[tile].bm - 1) / kTiles[tile].bm) * (n / kTiles[tile].bn);
 }
 
-bool split_fits(int tile, int n, int m, int n_split, size_t part_bytes) {
-  const int64_t tiles = tile_count(tile, n, m);
+int64_t tile_count(const Bf16x3Shape &t, int n, int m) {
+  return int64_t((m + t.bt - 1) / t.bt) * ((n + t.bw - 1) / t.bw);
+}
+
+bool parts_fit(int64_t tiles, int tile_floats, int n_split, size_t part_bytes) {
   return tiles <= kSplitCounters &&
-         static_cast<size_t>(tiles) * n_split * kTiles[tile].bm * kTiles[tile].bn * sizeof(float) <=
-             part_bytes;
+         static_cast<size_t>(tiles) * n_split * tile_floats * sizeof(float) <= part_bytes;
+}
+
+bool split_fits(int tile, int n, int m, int n_split, size_t part_bytes) {
+  if (tile >= kNumTiles) {
+    const Bf16x3Shape &t = kBf16x3[tile - kNumTiles];
+    return parts_fit(tile_count(t, n, m), t.bt * t.bw, n_split, part_bytes);
+  }
+  return parts_fit(tile_count(tile, n, m), kTiles[tile].bm * kTiles[tile].bn, n_split, part_bytes);
 }
 
 __global__ void zero_ints_kernel(int *p, int n) {
@@ -510,7 +542,7 @@ bool gemm_nt_supported(int64_t n_out, int64_t k, int64_t m) {
          k <= kMaxK && m <= INT_MAX / 2;
 }
 
-GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split) {
+GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, double *units) {
   const int n = static_cast<int>(n_out), mm = static_cast<int>(m);
   const int steps = static_cast<int>(k / BK);
   // the least estimated time; on a tie the larger tile, then fewer splits
@@ -530,10 +562,42 @@ GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split) {
       }
     }
   }
+  if (units) *units = best;
   return p;
 }
 
-// The tile shapes (tokens x outputs): 0 128 x 128, 1 64 x 64, 2 64 x 32,
+GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split) {
+  double best;
+  GemmPlan p = gemm_f32_plan(n_out, k, m, may_split, &best);
+  if (!gemm_bf16x3_supported(n_out, k, m)) return p;
+  const int n = static_cast<int>(n_out), mm = static_cast<int>(m);
+  const int steps = static_cast<int>(k / BK);
+  // the bf16-piece kernel where it promises to be faster and has at least as
+  // many K ranges as the F32 plan (each halving of a sum's length takes about
+  // 1.4 off its rounding error, and the pieces start 1.15 ahead)
+  const int f32_split = p.split;
+  double best_us = kBf16x3Margin * (kFixedUs + kUnitUs * best);
+  for (int i = 0; i < kNumBf16x3; ++i) {
+    const Bf16x3Shape &t = kBf16x3[i];
+    const int64_t tiles = tile_count(t, n, mm);
+    for (int sk = 1; sk <= (may_split ? kMaxSplit : 1); ++sk) {
+      if (sk > 1 && (steps < 2 * sk || !split_fits(kNumTiles + i, n, mm, sk, kSplitPartBytes))) break;
+      if (sk * t.groups < f32_split) continue;
+      const int64_t per_cu = (tiles * sk + kCUs - 1) / kCUs;
+      const int64_t rest = per_cu % t.res;
+      double us = static_cast<double>(per_cu / t.res) * t.us[t.res - 1];
+      if (rest) us += t.us[rest - 1];
+      us = t.fixed + us * steps / sk + (sk > 1 ? t.split + t.per_split * (sk - 1) : 0.0);
+      if (us < best_us) {
+        best_us = us;
+        p = GemmPlan{kNumTiles + i, sk};
+      }
+    }
+  }
+  return p;
+}
+
+// The F32 tile shapes (tokens x outputs): 0 128 x 128, 1 64 x 64, 2 64 x 32,
 // 3 32 x 64, 4 32 x 32; each a 2 x 2 grid of wavefronts.
 int gemm_nt_tile(int tile, int n_split, const float *w, const float *x, float *out,
                  const float *residual, int n, int kk, int mm, float *part, int *counters,
@@ -547,7 +611,9 @@ int gemm_nt_tile(int tile, int n_split, const float *w, const float *x, float *o
     case 2: return launch<2, 1, 2, 2>(w, x, out, residual, n, kk, mm, n_split, part, counters, s);
     case 3: return launch<1, 2, 2, 2>(w, x, out, residual, n, kk, mm, n_split, part, counters, s);
     case 4: return launch<1, 1, 2, 2>(w, x, out, residual, n, kk, mm, n_split, part, counters, s);
-    default: return -EINVAL;
+    default:
+      return gemm_bf16x3_tile(tile - kNumTiles, n_split, w, x, out, residual, n, kk, mm, part,
+                              counters, s);
   }
 }
 
@@ -589,7 +655,7 @@ extern "C" int ikv_bench_gemm_nt_tile_f32(const float *w, const float *x, float 
                                           size_t ws_bytes, void *stream) {
   if (!w || !x || !out || n_out <= 0 || k <= 0 || m <= 0) return -EINVAL;
   if (!ikv::gemm_nt_supported(n_out, k, m)) return -ENOTSUP;
-  if (tile < 0 || tile >= kNumTiles || n_split < 1) return -EINVAL;
+  if (tile < 0 || tile >= kNumTiles + kNumBf16x3 || n_split < 1) return -EINVAL;
   float *part = nullptr;
   int *counters = nullptr;
   if (n_split > 1) {
@@ -605,6 +671,15 @@ extern "C" int ikv_bench_gemm_nt_tile_f32(const float *w, const float *x, float 
 }
 
 extern "C" int ikv_bench_gemm_plan(int64_t n_out, int64_t k, int64_t m, int *tile, int *n_split) {
+  if (!tile || !n_split || n_out <= 0 || k <= 0 || m <= 0) return -EINVAL;
+  if (!ikv::gemm_nt_supported(n_out, k, m)) return -ENOTSUP;
+  const ikv::GemmPlan p = ikv::gemm_f32_plan(n_out, k, m, true, nullptr);
+  *tile = p.tile;
+  *n_split = p.split;
+  return 0;
+}
+
+extern "C" int ikv_bench_gemm_choice(int64_t n_out, int64_t k, int64_t m, int *tile, int *n_split) {
   if (!tile || !n_split || n_out <= 0 || k <= 0 || m <= 0) return -EINVAL;
   if (!ikv::gemm_nt_supported(n_out, k, m)) return -ENOTSUP;
   const ikv::GemmPlan p = ikv::gemm_plan(n_out, k, m, true);

@@ -163,6 +163,7 @@ BENCH_SIGNATURES = {
         _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int64, _c_int64, _c_int64, _c_void_p, _c_int,
                  _c_int, _c_void_p, _c_size_t, _c_void_p]),
     "ikv_bench_gemm_plan": (_c_int, [_c_int64, _c_int64, _c_int64, _c_void_p, _c_void_p]),
+    "ikv_bench_gemm_choice": (_c_int, [_c_int64, _c_int64, _c_int64, _c_void_p, _c_void_p]),
 }
 
 

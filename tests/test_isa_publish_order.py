@@ -101,6 +101,14 @@ def test_split_k_gemm_publishes_before_counting(tmp_path):
         check_publish_order(name, body)  # every thread stores its partial, one counts
 
 
+def test_split_k_piece_gemm_publishes_before_counting(tmp_path):
+    asm = device_asm(CSRC / "gemm_bf16x3.hip", tmp_path)
+    found = [(n, b) for n, b in functions(asm) if "gemm_bf16x3_kernel" in n]
+    assert len(found) == 4  # the four tile shapes
+    for name, body in found:
+        check_publish_order(name, body)
+
+
 def test_sampler_publishes_before_counting(tmp_path):
     asm = device_asm(CSRC / "model_ops.hip", tmp_path)
     found = [(n, b) for n, b in functions(asm) if "argmax_ws_kernel" in n]
