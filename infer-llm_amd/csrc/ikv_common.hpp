@@ -84,11 +84,15 @@ __device__ __forceinline__ double dpp64(double v) {
   const int hi = __builtin_amdgcn_mov_dpp(u.y, CTRL, 0xF, 0xF, false);
   return __builtin_bit_cast(double, make_int2(lo, hi));
 }
-__device__ __forceinline__ double half_wave_sum_f64(double v) {
+__device__ __forceinline__ double row16_sum_f64(double v) {
   v += dpp64<kDppXor1>(v);
   v += dpp64<kDppXor2>(v);
   v += dpp64<kDppHalfMirror>(v);
   v += dpp64<kDppMirror>(v);
+  return v;
+}
+__device__ __forceinline__ double half_wave_sum_f64(double v) {
+  v = row16_sum_f64(v);
   const uint2 u = __builtin_bit_cast(uint2, v);
   const auto lo = __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
   const auto hi = __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
@@ -154,10 +158,12 @@ constexpr float kLog2e = 1.4426950408889634f;
 // other order's). The doubles computed from S and S' by the same four
 // correctly rounded operations then differ by at most
 // (n_err / 2 + 8) * 2^-53 relative. This returns the float scale from S'
-// when every double within 64 times that of its value rounds to the same
+// when every double within twice that of its value rounds to the same
 // float, which makes it the reference's float bit for bit; it returns false
-// (about 2^-16 of rows; also for zero, infinite and NaN values) when the
-// caller must sum in index order instead.
+// (about 2^-17 of rows of 4096 floats, 2^-19 of 1024; also for infinite and
+// NaN values) when the caller must sum in index order instead. (64 times
+// that, as it was, sent one row of 4096 floats in 3000 to the index-order
+// sum, so nearly every norm of a few thousand rows waited for one.)
 __device__ __forceinline__ bool certified_rms_scale(double s_any, int dim, float eps, int n_err,
                                                     float &scale) {
   const double t = 1.0 / sqrt(s_any / static_cast<double>(dim) + static_cast<double>(eps));
@@ -170,7 +176,7 @@ __device__ __forceinline__ bool certified_rms_scale(double s_any, int dim, float
   const double nb = static_cast<double>(__uint_as_float(t >= fd ? bits + 1u : bits - 1u));
   const double mid = 0.5 * (fd + nb);
   const double rel = (0.5 * n_err + 8.0) * 0x1p-53;
-  if (fabs(mid - t) <= 64.0 * rel * t) return false;
+  if (fabs(mid - t) <= 2.0 * rel * t) return false;
   scale = f;
   return true;
 }
@@ -186,16 +192,39 @@ __device__ __forceinline__ float ordered_rms_scale(const float *row, int dim, fl
   return static_cast<float>(1.0 / sqrt(sum / static_cast<double>(dim) + static_cast<double>(eps)));
 }
 
+// The same by a whole wavefront: 64 floats at a time are loaded and squared
+// side by side and added one lane after the other (v_readlane), so the chain
+// holds a double add per float and no load. One lane walking a row of 4096
+// floats in memory took about 290 us, a load's latency every few floats.
+__device__ __forceinline__ float ordered_rms_scale_wave(const float *row, int dim, float eps,
+                                                        int lane) {
+  double sum = 0.0;
+  float next = lane < dim ? row[lane] : 0.f;
+  for (int i0 = 0; i0 < dim; i0 += 64) {
+    const float x = next;  // (zeros past the row add nothing)
+    if (i0 + 64 < dim) next = i0 + 64 + lane < dim ? row[i0 + 64 + lane] : 0.f;
+    const float sq = x * x;
+    uint2 d = __builtin_bit_cast(uint2, static_cast<double>(sq));
+    for (int q = 0; q < 4; ++q) {  // (a loop: this path is rare and its code in every norm)
+#pragma unroll
+      for (int l = 0; l < 16; ++l)
+        sum += __builtin_bit_cast(double, make_uint2(__builtin_amdgcn_readlane(d.x, l),
+                                                     __builtin_amdgcn_readlane(d.y, l)));
+      d.x = __shfl_down(d.x, 16, 64);
+      d.y = __shfl_down(d.y, 16, 64);
+    }
+  }
+  return static_cast<float>(1.0 / sqrt(sum / static_cast<double>(dim) + static_cast<double>(eps)));
+}
+
 // certified_rms_scale for a sum that every lane of the wave holds, else the
-// index-order sum by lane 0, broadcast (wave-uniform control flow).
+// index-order sum by the wave (wave-uniform control flow).
 __device__ __forceinline__ float certified_or_ordered_scale(double s_any, const float *row,
                                                             int dim, float eps, int n_err,
                                                             int lane) {
   float scale = 0.f;
   if (certified_rms_scale(s_any, dim, eps, n_err, scale)) return scale;
-  float seq = 0.f;
-  if (lane == 0) seq = ordered_rms_scale(row, dim, eps);
-  return __shfl(seq, 0, 64);
+  return ordered_rms_scale_wave(row, dim, eps, lane);
 }
 
 // RMSNorm scale float(1 / sqrt(sum/dim + eps)) of a row of dim floats
@@ -204,22 +233,25 @@ __device__ __forceinline__ float certified_or_ordered_scale(double s_any, const 
 // elements 256*j + 4*l + c (j ascending, c = 0..3), the 64 lane sums combine
 // in wave_sum_f64's tree (every lane gets the same bits), and the
 // scale is certified against the index-order sum (certified_rms_scale); when
-// it is not certain, lane 0 sums the row in index order (about 9 us for 1024
-// floats; rare) and every lane takes that.
+// it is not certain, the wave sums the row in index order.
+__device__ __forceinline__ double add_squares(double s, const float4 v) {
+  const float a = v.x * v.x, b = v.y * v.y, c = v.z * v.z, d = v.w * v.w;
+  s += static_cast<double>(a);
+  s += static_cast<double>(b);
+  s += static_cast<double>(c);
+  s += static_cast<double>(d);
+  return s;
+}
+// from the lanes' sums (row: for the index-order sum)
+__device__ __forceinline__ float rms_scale_of_lane_sums(double s, const float *row, int dim,
+                                                        float eps, int lane) {
+  return certified_or_ordered_scale(wave_sum_f64(s), row, dim, eps, (dim - 1) + dim / 64 + 5, lane);
+}
 __device__ __forceinline__ float rms_scale_strided(const float4 *row, int dim, float eps, int lane) {
   double s = 0.0;
 #pragma unroll 4
-  for (int j = 0; j < dim / 256; ++j) {
-    const float4 v = row[64 * j + lane];
-    const float a = v.x * v.x, b = v.y * v.y, c = v.z * v.z, d = v.w * v.w;
-    s += static_cast<double>(a);
-    s += static_cast<double>(b);
-    s += static_cast<double>(c);
-    s += static_cast<double>(d);
-  }
-  s = wave_sum_f64(s);
-  return certified_or_ordered_scale(s, reinterpret_cast<const float *>(row), dim, eps,
-                                    (dim - 1) + dim / 64 + 5, lane);
+  for (int j = 0; j < dim / 256; ++j) s = add_squares(s, row[64 * j + lane]);
+  return rms_scale_of_lane_sums(s, reinterpret_cast<const float *>(row), dim, eps, lane);
 }
 
 // ORs an IKV_STATUS_* bit into a caller's device status word (a vector

@@ -19,18 +19,19 @@
 // scale against the index-order sum (ikv::certified_rms_scale): the two sums
 // differ by a bounded amount, and when the double scale is farther than that
 // from a float rounding midpoint, both round to the same float. When it is
-// not (about 2^-16 of rows), one lane redoes the sum in index order. Every
+// not (about 2^-19 of rows of 1024 floats), the sum is redone in index order. Every
 // scale is therefore the reference's bit for bit.
-//  * rows shorter than kLongRow (the head_dim rows of qk-norm): half-wave per
-//    row, lane c adds elements c, c + 32, ..., then a xor butterfly;
+//  * rows shorter than kLongRow: half-wave per row, lane c adds elements c,
+//    c + 32, ..., then a xor butterfly; the head rows of qk-norm: each lane
+//    adds its four;
 //  * rows of kLongRow or more floats, a multiple of 256 (the model-width
 //    rows of attn_norm / ffn_norm / output_norm): one wavefront per row; lane
-//    l adds the squares of elements 256*j + 4*l + c (j ascending,
-//    c = 0..3), then the 64 lane sums combine in a xor butterfly
-//    (ikv::rms_scale_strided). The GEMV kernels that fold this norm into
-//    their input (ikv_model.h) use the same scale.
+//    l adds the squares of elements 256*j + 4*l + c (j ascending, the four c
+//    apart), then the lane sums combine. The GEMV kernels that fold this norm
+//    into their input (ikv_model.h) certify the same scale.
 //
-// Short rows: each workgroup is 4 wavefronts owning up to 16 rows. It issues
+// Head rows of 64, 128 or 256 floats with RoPE: head_rope_kernel below. Other
+// short rows: each workgroup is 4 wavefronts owning up to 16 rows. It issues
 // all of its row loads at once (coalesced, float4 when aligned) together with
 // the positions, norm weights and sin/cos rows of its first RoPE pairs, then
 // stages the rows in LDS (row stride dim+1 floats, so the per-lane row walks
@@ -44,6 +45,7 @@
 #include "../../include/ikv.h"
 
 #include <climits>
+#include <initializer_list>
 #include <vector>
 
 namespace {
@@ -249,29 +251,208 @@ __global__ __launch_bounds__(kRowThreads) void row_kernel(const float *__restric
 }
 
 // Model-width rows: one wavefront per row, lane-strided double sum (the
-// order described above), float4 loads and stores.
+// order described above), float4 loads and stores. Bound by memory with many
+// rows and by the latency of one row's loads with few, so rows of up to
+// 256 * NV floats are loaded once, all loads in flight together, and stay in
+// registers (NV = 0: longer rows, read twice). Graphs of 20 launches: 4096 rows
+// of 4096 floats 292 us (mostly one wave's index-order sum) -> 22.5 (5.9 TB/s),
+// 1024 rows 9.7 -> 7.3, one row 5.0 -> 3.5; 2048 rows of 1024 4.5 -> 4.2.
+template <int NV>
 __global__ __launch_bounds__(256) void long_row_norm_kernel(const float *__restrict__ x,
                                                             const float *__restrict__ w, float *out,
                                                             int64_t rows, int dim, float eps) {
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
+  const int nj = dim / 256;
   const float4 *xr = reinterpret_cast<const float4 *>(x + row * dim);
-  const float scale = ikv::rms_scale_strided(xr, dim, eps, lane);
   const float4 *w4 = reinterpret_cast<const float4 *>(w);
   float4 *o4 = reinterpret_cast<float4 *>(out + row * dim);
-  for (int j = lane; j < dim / 4; j += 64) {
-    const float4 v = xr[j];
-    const float4 g = w4[j];
-    const float a = v.x * scale, b = v.y * scale, c = v.z * scale, d = v.w * scale;
-    o4[j] = make_float4(a * g.x, b * g.y, c * g.z, d * g.w);
+  auto scaled = [](float4 v, float4 g, float s) {
+    const float a = v.x * s, b = v.y * s, c = v.z * s, d = v.w * s;
+    return make_float4(a * g.x, b * g.y, c * g.z, d * g.w);
+  };
+  if constexpr (NV > 0) {
+    // pieces past the row load its last one and count as zeros, so that no
+    // branch stands between the loads
+    float4 v[NV], g[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = xr[64 * min(j, nj - 1) + lane];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) g[j] = w4[64 * min(j, nj - 1) + lane];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};  // four chains of adds instead of one
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const float a = v[j].x * v[j].x, b = v[j].y * v[j].y, c = v[j].z * v[j].z, d = v[j].w * v[j].w;
+      const bool on = j < nj;
+      s[0] += on ? static_cast<double>(a) : 0.0;
+      s[1] += on ? static_cast<double>(b) : 0.0;
+      s[2] += on ? static_cast<double>(c) : 0.0;
+      s[3] += on ? static_cast<double>(d) : 0.0;
+    }
+    const float scale = ikv::rms_scale_of_lane_sums((s[0] + s[1]) + (s[2] + s[3]),
+                                                    reinterpret_cast<const float *>(xr), dim, eps, lane);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+      if (j < nj) o4[64 * j + lane] = scaled(v[j], g[j], scale);
+  } else {
+    const float scale = ikv::rms_scale_strided(xr, dim, eps, lane);
+    for (int j = lane; j < dim / 4; j += 64) o4[j] = scaled(xr[j], w4[j], scale);
   }
+}
+
+// Head rows of 64, 128 or 256 floats with RoPE (and qk-norm): LPR = dim / 4
+// lanes per row, lane c holding the pairs (2c, 2c + 1) of both halves, so a
+// row's rotation is lane-local and nothing goes through LDS or a barrier. A
+// wave owns R sets of 64 / LPR rows, all their loads in flight together.
+// Bound by memory with many rows (4096 tokens x 32 heads of 128: 134 MB) and
+// by the chain position -> angles -> rotation with few. With R = 4 the four
+// sums of a lane's rows are certified by the four lanes of a quad at once
+// (the double square root and divisions of every row in every lane cost as
+// much as the memory). Measured against row_kernel in graphs of 20 launches:
+// 4096 tokens x 32 heads of 128 50.1 -> 23.3 us (5.8 TB/s), 2048 x 16 17.1 ->
+// 7.9, 37 x 16 5.9 -> 2.5, one token 5.5 -> 2.2; 1500 x 12 of 64 8.0 -> 3.7.
+template <int LPR, int R, bool NORM>
+__global__ __launch_bounds__(256) void head_rope_kernel(
+    const float *__restrict__ x, const float *__restrict__ w, float *out,
+    const int32_t *__restrict__ pos, unsigned rows, float eps, unsigned n_heads,
+    const float *__restrict__ sin_tab, const float *__restrict__ cos_tab, int64_t n_ctx,
+    int *status) {
+  constexpr int DIM = 4 * LPR, HD = 2 * LPR;
+  constexpr unsigned SETS = 64 / LPR;  // rows per set
+  const int lane = threadIdx.x & 63;
+  const int c = lane % LPR;
+  const unsigned row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (SETS * R) + lane / LPR;
+  float2 lo[R], hi[R], cs[R], sn[R];
+  int32_t p[R];
+  unsigned row[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) row[r] = min(row0 + SETS * r, rows - 1);  // past the end: not stored
+#pragma unroll
+  for (int r = 0; r < R; ++r) p[r] = pos[row[r] / n_heads];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const float2 *xr = reinterpret_cast<const float2 *>(x + static_cast<size_t>(row[r]) * DIM);
+    lo[r] = xr[c];
+    hi[r] = xr[LPR + c];
+  }
+  float2 wl = make_float2(0.f, 0.f), wh = wl;
+  if constexpr (NORM) {
+    wl = reinterpret_cast<const float2 *>(w)[c];
+    wh = reinterpret_cast<const float2 *>(w)[LPR + c];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool in = p[r] >= 0 && p[r] < n_ctx;
+    const size_t at = static_cast<size_t>(in ? p[r] : 0) * HD;
+    cs[r] = reinterpret_cast<const float2 *>(cos_tab + at)[c];
+    sn[r] = reinterpret_cast<const float2 *>(sin_tab + at)[c];
+  }
+  if constexpr (NORM) {
+    double sum[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double s = ikv::add_squares(0.0, make_float4(lo[r].x, lo[r].y, hi[r].x, hi[r].y));
+      sum[r] = LPR == 16   ? ikv::row16_sum_f64(s)
+               : LPR == 32 ? ikv::half_wave_sum_f64(s)
+                           : ikv::wave_sum_f64(s);
+    }
+    // lane of quad position k certifies row set k (R == 1: every lane its own)
+    double mine = sum[0];
+    if constexpr (R == 4) {
+      const int k = lane & 3;
+      mine = k == 0 ? sum[0] : k == 1 ? sum[1] : k == 2 ? sum[2] : sum[3];
+    }
+    float scale = -1.f;  // (a certified scale is positive)
+    if (!ikv::certified_rms_scale(mine, DIM, eps, (DIM - 1) + 4 + 6, scale)) scale = -1.f;
+    float sc[R];
+    if constexpr (R == 4) {
+      sc[0] = ikv::dpp<0x00>(scale);  // quad_perm [k, k, k, k]
+      sc[1] = ikv::dpp<0x55>(scale);
+      sc[2] = ikv::dpp<0xAA>(scale);
+      sc[3] = ikv::dpp<0xFF>(scale);
+    } else {
+      sc[0] = scale;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      // rows in doubt: the wave sums each in index order
+      for (unsigned long long todo = __builtin_amdgcn_ballot_w64(sc[r] < 0.f); todo != 0;) {
+        const int src = __builtin_ctzll(todo);
+        const unsigned rr = __builtin_amdgcn_readlane(row[r], src);
+        const float s = ikv::ordered_rms_scale_wave(x + static_cast<size_t>(rr) * DIM, DIM, eps, lane);
+        if (lane / LPR == src / LPR) sc[r] = s;
+        todo &= ~((LPR == 64 ? ~0ull : (1ull << (LPR % 64)) - 1) << (src / LPR * LPR));
+      }
+      const float a = lo[r].x * sc[r], b = lo[r].y * sc[r], d = hi[r].x * sc[r], e = hi[r].y * sc[r];
+      lo[r] = make_float2(a * wl.x, b * wl.y);
+      hi[r] = make_float2(d * wh.x, e * wh.y);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (row0 + SETS * r >= rows) continue;
+    float2 o0 = make_float2(0.f, 0.f), o1 = o0;
+    if (p[r] < 0 || p[r] >= n_ctx) {
+      ikv::raise_status(status, IKV_STATUS_POSITION);
+    } else {
+      const float a0 = lo[r].x * cs[r].x, b0 = hi[r].x * sn[r].x;
+      const float a1 = lo[r].y * cs[r].y, b1 = hi[r].y * sn[r].y;
+      const float e0 = lo[r].x * sn[r].x, f0 = hi[r].x * cs[r].x;
+      const float e1 = lo[r].y * sn[r].y, f1 = hi[r].y * cs[r].y;
+      o0 = make_float2(a0 - b0, a1 - b1);
+      o1 = make_float2(e0 + f0, e1 + f1);
+    }
+    float2 *orow = reinterpret_cast<float2 *>(out + static_cast<size_t>(row[r]) * DIM);
+    orow[c] = o0;
+    orow[LPR + c] = o1;
+  }
+}
+
+bool aligned8(std::initializer_list<const void *> ptrs) {
+  for (const void *q : ptrs)
+    if (reinterpret_cast<uintptr_t>(q) & 7) return false;
+  return true;
+}
+
+// R = 4 row sets per wave once that still gives every SIMD two waves.
+constexpr int64_t kManyRows = 8 * 2048;
+
+template <bool NORM>
+int launch_heads(const float *x, const float *w, float *out, const int32_t *pos, int64_t rows,
+                 int dim, float eps, int n_heads, const float *sin_tab, const float *cos_tab,
+                 int64_t n_ctx, int *status, void *stream) {
+  const int sets = 256 / dim;  // rows of one set of a wave
+  const int r = rows * dim >= kManyRows * 128 ? 4 : 1;
+  const unsigned per_block = 4u * static_cast<unsigned>(sets * r);
+  const unsigned blocks = (static_cast<unsigned>(rows) + per_block - 1) / per_block;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define IKV_HEADS(LPR, RR)                                                                       \
+  head_rope_kernel<LPR, RR, NORM><<<blocks, 256, 0, s>>>(x, w, out, pos,                         \
+                                                         static_cast<unsigned>(rows), eps,       \
+                                                         static_cast<unsigned>(n_heads), sin_tab, \
+                                                         cos_tab, n_ctx, status)
+  if (dim == 64) {
+    if (r == 4) IKV_HEADS(16, 4); else IKV_HEADS(16, 1);
+  } else if (dim == 128) {
+    if (r == 4) IKV_HEADS(32, 4); else IKV_HEADS(32, 1);
+  } else {
+    if (r == 4) IKV_HEADS(64, 4); else IKV_HEADS(64, 1);
+  }
+#undef IKV_HEADS
+  return ikv::launch_status();
 }
 
 template <bool NORM, bool ROPE>
 int launch_rows(const float *x, const float *w, float *out, const int32_t *pos, int64_t rows,
                 int dim, float eps, int n_heads, const float *sin_tab, const float *cos_tab,
                 int64_t n_ctx, int *status, void *stream) {
+  if constexpr (ROPE) {
+    if ((dim == 64 || dim == 128 || dim == 256) && rows <= INT_MAX &&
+        aligned8({x, w, out, sin_tab, cos_tab}))
+      return launch_heads<NORM>(x, w, out, pos, rows, dim, eps, n_heads, sin_tab, cos_tab, n_ctx,
+                                status, stream);
+  }
   const int rpb = rows_per_block(dim);
   const int64_t blocks = (rows + rpb - 1) / rpb;
   if (blocks > INT_MAX) return -EOVERFLOW;
@@ -295,7 +476,10 @@ extern "C" int ikv_rms_norm_f32(const float *x, const float *w, float *out, int6
       ikv::aligned16(out)) {
     const int64_t blocks = (rows + 3) / 4;
     if (blocks > INT_MAX) return -EOVERFLOW;
-    long_row_norm_kernel<<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
+    const auto kernel = dim <= 1024   ? long_row_norm_kernel<4>
+                        : dim <= 4096 ? long_row_norm_kernel<16>
+                                      : long_row_norm_kernel<0>;
+    kernel<<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
         x, w, out, rows, static_cast<int>(dim), eps);
     return ikv::launch_status();
   }
