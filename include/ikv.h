@@ -214,12 +214,15 @@ int64_t ikv_attn_decode_replay_limit(int n_head, int n_head_kv, int head_dim, in
 /* ---------------------------------------------------------------------
  * Prefill / general attention, n_q >= 1 query tokens, causal: key j is
  * visible to query t iff j <= n_past + t (src/backends/cpu_backend.cpp:578,
- * src/kernels/cuda/kernel_f32.cu:346). F32 MFMA tiles; K/V tiles staged in
- * LDS and shared by the n_head/n_head_kv query heads of a KV head.
+ * src/kernels/cuda/kernel_f32.cu:346). MFMA tiles, F32 or (longer prompts)
+ * bf16 with every float split into three exact bf16 pieces; K/V tiles staged
+ * in LDS and shared by the n_head/n_head_kv query heads of a KV head.
  * Replaces compute_flash_attn for n_q > 1. Needs no workspace.
  * The MFMA kernel takes head_dim 128 with n_head/n_head_kv 1, 2, 4 or 8;
  * any other head_dim in [1, 512] and any n_head that n_head_kv divides run
- * the generic path (decode above). Larger head_dim: -ENOTSUP. The MFMA
+ * the generic path (decode above), of which the prompts of 96 keys and more
+ * with head_dim a multiple of 4 up to 128 and 16-byte aligned operands use
+ * the bf16 MFMA kernel too. Larger head_dim: -ENOTSUP. The MFMA
  * kernel's shapes with n_head_kv > 65536: -EOVERFLOW.
  * ------------------------------------------------------------------- */
 int ikv_attn_prefill_f32(const float *q, const float *k, const float *v, float *out, int n_head,

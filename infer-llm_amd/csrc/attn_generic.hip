@@ -6,7 +6,8 @@
 // key j is visible to query t iff j <= n_past + t and j < n_kv; q head h
 // reads KV head h / (n_head / n_head_kv).
 //
-// Prompts (and any n_q): a workgroup of 4 wavefronts owns 16 query rows of
+// Prompts with long rows and head_dim a multiple of 4 up to 128 go to
+// attn_bf16x3.hip. Others (and any n_q): a workgroup of 4 wavefronts owns 16 query rows of
 // one KV head g (row r = token * G + query head in the group, so a block of
 // rows covers every query head of its tokens and each K / V tile serves all
 // of them). Key tiles of KT rows (64 keys for head_dim <= 128, fewer for
@@ -21,6 +22,7 @@
 // all 4 rows.
 //
 // One query token (a decode step): the split form below.
+#include "attn_bf16x3.hpp"
 #include "attn_generic.hpp"
 #include "ikv_common.hpp"
 
@@ -41,6 +43,12 @@ __device__ __forceinline__ int64_t key_row(const ikv::Pages &pg, bool paged, int
   }
   return static_cast<int64_t>(blk) * pg.bt + (j - b * pg.bt);
 }
+
+// Keys of the longest row from which attn_bf16x3 takes a prompt: 12 heads of
+// 64 over 4, 64 tokens 7.4 us here against 8.3 there, 128 tokens 11.0 against
+// 10.5, 37 tokens behind 1000 65 against 28; heads of 80, 100 tokens 16.6
+// against 14.5.
+constexpr int64_t kPiecesMinKeys = 96;
 
 constexpr int kTileRowsPerWave = 4;  // 8 measured slower (fewer workgroups, more registers)
 constexpr int kTileRows = 4 * kTileRowsPerWave;  // query rows per workgroup
@@ -429,6 +437,9 @@ int attn_generic(const float *q, const float *k, const float *v, const Pages *pa
   if (!generic_attn_shape(n_head, n_head_kv, head_dim)) return -ENOTSUP;
   if (n_q < 0 || n_kv <= 0 || n_past < 0) return -EINVAL;
   if (n_q > INT_MAX / n_head || n_kv > INT_MAX / 2 || n_past > INT_MAX / 2) return -EOVERFLOW;
+  if (std::min(n_kv, n_past + n_q) >= kPiecesMinKeys &&
+      attn_bf16x3_supported(q, k, v, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past))
+    return attn_bf16x3(q, k, v, pages, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past, scale, s);
   if (!(scale > 0.0f)) scale = 1.0f / sqrtf(static_cast<float>(head_dim));
   const int dl = head_dim <= 64 ? 1 : head_dim <= 128 ? 2 : head_dim <= 256 ? 4 : 8;
   const int64_t rows = n_q * (n_head / n_head_kv);

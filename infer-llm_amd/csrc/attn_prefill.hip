@@ -1,5 +1,7 @@
 // attn_prefill.hip — causal GQA flash attention for n_q >= 1 query tokens on
-// F32 MFMA (v_mfma_f32_16x16x4_f32), never materialising the score matrix.
+// F32 MFMA (v_mfma_f32_16x16x4_f32), never materialising the score matrix:
+// prompts too short for attn_bf16x3.hip, to which prefill_common sends the
+// others.
 //
 // Replaces CUDA_F32::compute_flash_attn for prefill (reference
 // src/kernels/cuda/kernel_f32.cu:452-511), which allocated Hq*n_q*n_kv floats
@@ -56,6 +58,7 @@
 //     of tiles needs only the waves of one group to agree: each group passes
 //     an LDS arrival counter instead of the workgroup barrier, and the
 //     groups drift apart (P = 2048: 144.4 -> 141.4 us, alternated runs).
+#include "attn_bf16x3.hpp"
 #include "attn_generic.hpp"
 #include "coherent.hpp"
 #include "ikv_common.hpp"
@@ -561,6 +564,16 @@ int prefill_common(const float *q, const float *k, const float *v, const ikv_kv_
   if (!(scale > 0.0f)) scale = 1.0f / sqrtf(static_cast<float>(head_dim));
   const float sl2 = scale * ikv::kLog2e;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // More 16-row blocks than CUs, over more than 256 keys: the bf16-piece
+  // kernel. Up to one block per CU this kernel's one-wave groups win (0.6B
+  // heads, 256 tokens 11.4 us against 20.9, 64 tokens behind 1000 26 against
+  // 53), and so do its larger blocks on short rows (64 heads, 200 tokens 19.1
+  // against 21.5); past both, 300 tokens 26.4 against 24.1 us, 2048 150
+  // against 122.
+  const int64_t row_blocks = (n_q * G + 15) / 16;
+  if (row_blocks * n_head_kv > kCUs && std::min(n_kv, n_past + n_q) > 256 &&
+      ikv::attn_bf16x3_supported(q, k, v, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past))
+    return ikv::attn_bf16x3(q, k, v, pg, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past, scale, s);
   const int nq = static_cast<int>(n_q), nk = static_cast<int>(n_kv), np = static_cast<int>(n_past);
   switch (G) {
     case 1: launch<1>(q, k, v, out, n_head_kv, nq, nk, np, sl2, pg, s); break;

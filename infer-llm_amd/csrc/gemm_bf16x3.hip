@@ -56,61 +56,20 @@
 // slower: it shares the matrix pipe), load instructions over 16 rows x 64
 // bytes with lane swaps (4-7% slower when power-bound, equal otherwise), two
 // steps of loads in flight (equal).
+#include "bf16x3.hpp"
 #include "coherent.hpp"
 #include "gemm.hpp"
 #include "ikv_common.hpp"
 
 #include <climits>
-#include <type_traits>
 
 namespace {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+using namespace ikv::pieces;
 
 constexpr int BK = 32;      // columns per step: one MFMA's contraction
 constexpr int kXcds = 8;
 constexpr int kGroupT = 8;   // token tiles per group of the tile order
-constexpr int kSplitOps = 44;  // VALU instructions of split8
-// Sums that are all below this may come from inputs below 2^-109, whose last
-// pieces fall off bf16's range (an error of at most 2^-134 of the other
-// factor, nothing beside a larger sum).
-constexpr float kTinySum = 0x1p-64f;
-
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(f);
-  }
-}
-
-// The three bf16 pieces of 8 floats: x = h + m + l exactly.
-struct Pieces {
-  bf16x8 p[3];
-};
-__device__ __forceinline__ void split2(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
-  h = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
-  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
-  m = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{ra, rb}, bf16x2));
-  const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
-  l = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
-}
-__device__ __forceinline__ Pieces split8(floatx4 u, floatx4 v) {
-  uintx4 h, m, l;
-  unsigned a, b, c;
-  split2(u[0], u[1], a, b, c); h[0] = a; m[0] = b; l[0] = c;
-  split2(u[2], u[3], a, b, c); h[1] = a; m[1] = b; l[1] = c;
-  split2(v[0], v[1], a, b, c); h[2] = a; m[2] = b; l[2] = c;
-  split2(v[2], v[3], a, b, c); h[3] = a; m[3] = b; l[3] = c;
-  return Pieces{{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m),
-                 __builtin_bit_cast(bf16x8, l)}};
-}
-
 template <int TM, int TN, int WM, int KG, int MINW>
 __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
     const float *__restrict__ w, const float *__restrict__ x, float *out, const float *residual,
@@ -243,14 +202,13 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
           load_w(v, s + 2);
         }
       }
-      constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};  // small terms first
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int p = 0; p < 6; ++p)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[P][i][h].p[pa[p]], bc[h][pb[p]],
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[P][i][h].p[kPieceA[p]], bc[h][kPieceB[p]],
                                                                  acc[i][j], 0, 0, 0);
       if constexpr (hi > lo) {
         constexpr int NM = 12 * TM;
