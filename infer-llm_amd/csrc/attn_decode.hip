@@ -1049,9 +1049,9 @@ size_t generic_ws_bytes(int n_head, int n_head_kv, int head_dim, int64_t n_kv) {
 
 // A decode step on the generic attention path, for head sizes and query
 // groupings the decode kernel does not take: the prologue (qk-RMSNorm + RoPE
-// of the new token, into the workspace) and the append run as the separate
-// kernels, then the attention of the one query over n_kv keys. No replay
-// form (-ENOTSUP).
+// of the new token) and the append inside the attention's first launch where
+// generic_decode_folds takes them, else as the separate kernels (the rotated
+// rows into the workspace) before it. No replay form (-ENOTSUP).
 int decode_generic(const float *q, float *k_cache, float *v_cache, const float *k_new,
                    const float *v_new, float *out, int n_head, int n_head_kv, int head_dim,
                    int64_t n_kv, float scale, void *workspace, size_t workspace_bytes,
@@ -1061,9 +1061,30 @@ int decode_generic(const float *q, float *k_cache, float *v_cache, const float *
   if (n_kv > INT_MAX / 2) return -EOVERFLOW;
   const size_t row_bytes = sizeof(float) * static_cast<size_t>(n_head_kv) * head_dim;
   if (k_new && pages && row_bytes % 16 != 0) return -ENOTSUP;
+  // the split partials come after the room for the prologue's rows (a smaller
+  // or no workspace runs the one-workgroup-per-head form)
+  const size_t pro_bytes = generic_pro_bytes(n_head, n_head_kv, head_dim);
+  void *split_ws = nullptr;
+  size_t split_bytes = 0;
+  if (workspace && workspace_bytes > pro_bytes) {
+    split_ws = static_cast<char *>(workspace) + pro_bytes;
+    split_bytes = workspace_bytes - pro_bytes;
+  }
+  ikv::DecodeNew fold;
+  if (pro)
+    fold = {pro->q_norm_w, pro->k_norm_w, pro->eps,   pro->pos,
+            pro->sin_tab,  pro->cos_tab,  pro->n_ctx, pro->status};
+  auto folds = [&](const ikv::DecodeNew *f) {
+    return ikv::generic_decode_folds(q, k_cache, v_cache, k_new, v_new, pg, n_head, n_head_kv,
+                                     head_dim, n_kv, split_ws, split_bytes, f);
+  };
+  auto folded = [&](const ikv::DecodeNew *f) {
+    return ikv::attn_generic_decode_folded(q, k_cache, v_cache, k_new, v_new, pg, out, n_head,
+                                           n_head_kv, head_dim, n_kv, scale, split_ws, f, s);
+  };
+  if (pro && folds(&fold)) return folded(&fold);
   if (pro) {
-    if (!workspace || workspace_bytes < generic_pro_bytes(n_head, n_head_kv, head_dim))
-      return -EINVAL;
+    if (!workspace || workspace_bytes < pro_bytes) return -EINVAL;
     float *q_rot = static_cast<float *>(workspace);
     float *k_rot = reinterpret_cast<float *>(
         static_cast<char *>(workspace) +
@@ -1078,6 +1099,7 @@ int decode_generic(const float *q, float *k_cache, float *v_cache, const float *
     q = q_rot;
     k_new = k_rot;
   }
+  if (folds(nullptr)) return folded(nullptr);
   if (k_new) {
     int rc;
     if (pages) {
@@ -1089,15 +1111,6 @@ int decode_generic(const float *q, float *k_cache, float *v_cache, const float *
       if (!rc) rc = ikv_append_f32(v_cache + at, v_new, 1, row_bytes, s);
     }
     if (rc) return rc;
-  }
-  // the split form's partials after the prologue's rows (a smaller or no
-  // workspace runs the one-workgroup-per-head form)
-  const size_t pro_bytes = generic_pro_bytes(n_head, n_head_kv, head_dim);
-  void *split_ws = nullptr;
-  size_t split_bytes = 0;
-  if (workspace && workspace_bytes > pro_bytes) {
-    split_ws = static_cast<char *>(workspace) + pro_bytes;
-    split_bytes = workspace_bytes - pro_bytes;
   }
   return ikv::attn_generic_decode(q, k_cache, v_cache, pg, out, n_head, n_head_kv, head_dim, n_kv,
                                   scale, split_ws, split_bytes, s);

@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <initializer_list>
 
 namespace {
 
@@ -362,38 +363,270 @@ __global__ __launch_bounds__(kSplitWaves * 64) void generic_split_kernel(
 
 // out[head][d] = sum_s e_s O_s[d] / sum_s e_s L_s, e_s = 2^(M_s - max_s M_s):
 // one workgroup per query head. Wave 0 forms the weights (lanes over splits)
-// and the sum; then every thread takes output dims and adds the splits'
-// parts in split order.
+// and the sum; the threads take output dims, and where a head has at most
+// 128 of them several threads share a dim, each taking a run of the splits,
+// the runs added in order. All latency: a thread's first kMergeAhead partials
+// load while wave 0 forms the weights (40 splits of 64 dims 4.1 -> 3.7 us).
 constexpr int kMergeThreads = 256;
+constexpr int kMergeAhead = 16;
 __global__ __launch_bounds__(kMergeThreads) void generic_merge_kernel(
     const float *__restrict__ part_ml, const float *__restrict__ part_o, float *__restrict__ out,
     int dim, int n_splits) {
+  constexpr int kPerLane = kSplitTargetWgs / 64;
   __shared__ float s_e[kSplitTargetWgs];
   __shared__ float s_L;
+  __shared__ float s_part[kMergeThreads];
   const int head = blockIdx.x;
   const size_t rec0 = static_cast<size_t>(head) * n_splits;
+  const int runs = dim <= 64 ? 4 : dim <= 128 ? 2 : 1;
+  const int per = kMergeThreads / runs, r = threadIdx.x / per;
+  const int lo = r * n_splits / runs, hi = (r + 1) * n_splits / runs;
+  float a[kMergeAhead];
+  auto load = [&](int d, int sp0) {
+#pragma unroll
+    for (int u = 0; u < kMergeAhead; ++u) {
+      a[u] = 0.f;
+      if (d < dim && sp0 + u < hi) a[u] = part_o[(rec0 + sp0 + u) * dim + d];
+    }
+  };
+  load(threadIdx.x % per, lo);
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    float M = -INFINITY;
-    for (int sp = lane; sp < n_splits; sp += 64) M = fmaxf(M, part_ml[2 * (rec0 + sp)]);
+    float2 ml[kPerLane];
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+      const int sp = lane + 64 * i;
+      ml[i] = make_float2(-INFINITY, 0.f);
+      if (sp < n_splits) ml[i] = reinterpret_cast<const float2 *>(part_ml)[rec0 + sp];
+    }
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) M = fmaxf(M, ml[i].x);
     M = ikv::wave_max(M);
-    float L = 0.f;
-    for (int sp = lane; sp < n_splits; sp += 64) {
-      const float ms = part_ml[2 * (rec0 + sp)];
-      const float e = ms == -INFINITY ? 0.f : ikv::fast_exp2(ms - M);
-      s_e[sp] = e;
-      L = fmaf(e, part_ml[2 * (rec0 + sp) + 1], L);
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+      const float e = ml[i].x == -INFINITY ? 0.f : ikv::fast_exp2(ml[i].x - M);
+      s_e[lane + 64 * i] = e;
+      L = fmaf(e, ml[i].y, L);
     }
     L = ikv::wave_sum(L);
     if (lane == 0) s_L = L;
   }
   __syncthreads();
   const float inv = 1.0f / s_L;
-  for (int d = threadIdx.x; d < dim; d += kMergeThreads) {
+  auto run = [&](int d) {
     float O = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < n_splits; ++sp) O = fmaf(s_e[sp], part_o[(rec0 + sp) * dim + d], O);
-    out[static_cast<size_t>(head) * dim + d] = O * inv;
+    for (int sp = lo; sp < hi; sp += kMergeAhead) {
+      if (sp != lo) load(d, sp);
+#pragma unroll
+      for (int u = 0; u < kMergeAhead; ++u)
+        if (sp + u < hi) O = fmaf(s_e[sp + u], a[u], O);
+    }
+    return O;
+  };
+  if (runs > 1) {
+    const int d = threadIdx.x % per;
+    s_part[threadIdx.x] = run(d);
+    __syncthreads();
+    if (r == 0 && d < dim) {
+      float O = s_part[d];
+      for (int i = 1; i < runs; ++i) O += s_part[i * per + d];
+      out[static_cast<size_t>(head) * dim + d] = O * inv;
+    }
+    return;
+  }
+  for (int d = threadIdx.x; d < dim; d += kMergeThreads) {
+    if (d != static_cast<int>(threadIdx.x)) load(d, lo);
+    out[static_cast<size_t>(head) * dim + d] = run(d) * inv;
+  }
+}
+
+// The split decode for rows of 16-byte pieces: head_dim a multiple of 4 up to
+// 256, at most 8 query heads per KV head. LPK lanes (a power of two >= dim / 4)
+// hold a key's row, a float4 each, so a wave scores 64 / LPK keys at once and a
+// score's sum takes log2(LPK) lane steps for all of them (generic_split_kernel
+// spends a 64-lane sum per key and head: its sums were most of its time). Each
+// lane group keeps its own softmax state; the states of the workgroup's 4
+// waves meet in LDS. The new token is folded in: with k_new, the split that
+// holds key n_kv - 1 takes its rows from there and writes them to the caches,
+// and with PRO every split first forms its rotated q rows (and that one the k
+// row), with the operations of head_rope_kernel, while its first keys are in
+// flight. Latency-bound at these sizes, hence one launch for what took five:
+// 12 heads of 64 over 4 at 2500 keys, with qk-norm + RoPE, 21.1 us in five
+// launches before, 6.4 here.
+template <int LPK, int GM, bool PRO>
+__global__ __launch_bounds__(256) void decode_rows_kernel(
+    const float *__restrict__ q, float *__restrict__ k, float *__restrict__ v,
+    const float *__restrict__ k_new, const float *__restrict__ v_new, float *__restrict__ part_ml,
+    float *__restrict__ part_o, int n_head_kv, int G, int dim, int n_kv, int keys_per_split,
+    int n_splits, float scale_log2, bool paged, ikv::Pages pg, ikv::DecodeNew pro) {
+  constexpr int KPW = 64 / LPK;            // keys a wave scores at once
+  constexpr int U = LPK == 16 ? 4 : 8;     // of them in flight
+  constexpr int STATES = 4 * KPW;
+  __shared__ __attribute__((aligned(16))) float s_q[GM * 4 * LPK], s_kn[4 * LPK], s_vn[4 * LPK];
+  __shared__ float s_m[STATES][GM], s_l[STATES][GM];
+  __shared__ __attribute__((aligned(16))) float s_o[STATES][GM][4 * LPK];
+  const int g = static_cast<int>(blockIdx.x) % n_head_kv;
+  const int split = static_cast<int>(blockIdx.x) / n_head_kv;
+  const int t_begin = split * keys_per_split;
+  const int t_end = min(n_kv, t_begin + keys_per_split);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane % LPK, state = wave * KPW + lane / LPK;
+  const bool on = 4 * c < dim;
+  const size_t tok_stride = static_cast<size_t>(n_head_kv) * dim;
+  const size_t at = static_cast<size_t>(g) * dim + 4 * c;
+  const bool newest = k_new && t_end == n_kv;  // this split holds the new token
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+
+  float4 kr[U], vr[U];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + STATES * u;
+      const int64_t row = key_row(pg, paged, j < t_end ? j : t_begin);
+      kr[u] = vr[u] = zero;
+      if (on && j < t_end) {
+        kr[u] = *reinterpret_cast<const float4 *>(k + row * tok_stride + at);
+        vr[u] = *reinterpret_cast<const float4 *>(v + row * tok_stride + at);
+      }
+    }
+  };
+  load(t_begin + state);
+
+  if constexpr (PRO) {
+#pragma clang fp contract(off)
+    constexpr int HD = 2 * LPK;  // dim == 4 LPK; lane c holds the pairs (2c, 2c + 1) of both halves
+    const int32_t p = pro.pos[0];
+    const bool in = p >= 0 && p < pro.n_ctx;
+    const size_t ang = static_cast<size_t>(in ? p : 0) * HD;
+    const float2 cs = reinterpret_cast<const float2 *>(pro.cos_tab + ang)[c];
+    const float2 sn = reinterpret_cast<const float2 *>(pro.sin_tab + ang)[c];
+    const int rows = G + (newest ? 1 : 0);  // row G: the key
+    for (int r0 = 0; r0 < rows; r0 += STATES) {
+      const int r = min(r0 + state, rows - 1);
+      const float *x = r < G ? q + (static_cast<size_t>(g) * G + r) * dim : k_new + static_cast<size_t>(g) * dim;
+      const float *w = r < G ? pro.q_norm_w : pro.k_norm_w;
+      float2 lo = reinterpret_cast<const float2 *>(x)[c], hi = reinterpret_cast<const float2 *>(x)[LPK + c];
+      const float2 wl = reinterpret_cast<const float2 *>(w)[c], wh = reinterpret_cast<const float2 *>(w)[LPK + c];
+      const double sq = ikv::add_squares(0.0, make_float4(lo.x, lo.y, hi.x, hi.y));
+      const double sum = LPK == 16   ? ikv::row16_sum_f64(sq)
+                         : LPK == 32 ? ikv::half_wave_sum_f64(sq)
+                                     : ikv::wave_sum_f64(sq);
+      float sc = -1.f;
+      if (!ikv::certified_rms_scale(sum, 4 * LPK, pro.eps, (4 * LPK - 1) + 4 + 6, sc)) sc = -1.f;
+      for (unsigned long long todo = __builtin_amdgcn_ballot_w64(sc < 0.f); todo != 0;) {
+        const int src = __builtin_ctzll(todo);
+        const int rr = __builtin_amdgcn_readlane(r, src);
+        const float *xr = rr < G ? q + (static_cast<size_t>(g) * G + rr) * dim : k_new + static_cast<size_t>(g) * dim;
+        const float sx = ikv::ordered_rms_scale_wave(xr, 4 * LPK, pro.eps, lane);
+        if (lane / LPK == src / LPK) sc = sx;
+        todo &= ~((LPK == 64 ? ~0ull : (1ull << (LPK % 64)) - 1) << (src / LPK * LPK));
+      }
+      const float a0 = lo.x * sc, a1 = lo.y * sc, b0 = hi.x * sc, b1 = hi.y * sc;
+      const float x0 = a0 * wl.x, x1 = a1 * wl.y, y0 = b0 * wh.x, y1 = b1 * wh.y;
+      const float m0 = x0 * cs.x, n0 = y0 * sn.x, m1 = x1 * cs.y, n1 = y1 * sn.y;
+      const float e0 = x0 * sn.x, f0 = y0 * cs.x, e1 = x1 * sn.y, f1 = y1 * cs.y;
+      float *dst = r < G ? s_q + r * 4 * LPK : s_kn;
+      reinterpret_cast<float2 *>(dst)[c] = in ? make_float2(m0 - n0, m1 - n1) : make_float2(0.f, 0.f);
+      reinterpret_cast<float2 *>(dst)[LPK + c] = in ? make_float2(e0 + f0, e1 + f1) : make_float2(0.f, 0.f);
+    }
+    if (!in && newest && threadIdx.x == 0) ikv::raise_status(pro.status, IKV_STATUS_POSITION);
+  } else {
+    for (int i = threadIdx.x; i < G * dim; i += 256)
+      s_q[i / dim * 4 * LPK + i % dim] = q[static_cast<size_t>(g) * G * dim + i];
+    if (newest)
+      for (int i = threadIdx.x; i < dim; i += 256) s_kn[i] = k_new[static_cast<size_t>(g) * dim + i];
+  }
+  if (newest)
+    for (int i = threadIdx.x; i < dim; i += 256) s_vn[i] = v_new[static_cast<size_t>(g) * dim + i];
+  __syncthreads();
+  if (newest && threadIdx.x < LPK && on) {  // the append
+    const int64_t row = key_row(pg, paged, n_kv - 1);
+    if (!paged || ikv::page_ok(pg, n_kv - 1)) {
+      *reinterpret_cast<float4 *>(k + row * tok_stride + at) = *reinterpret_cast<const float4 *>(s_kn + 4 * c);
+      *reinterpret_cast<float4 *>(v + row * tok_stride + at) = *reinterpret_cast<const float4 *>(s_vn + 4 * c);
+    }
+  }
+
+  float4 qv[GM], o[GM];
+  float m[GM], l[GM];
+#pragma unroll
+  for (int h = 0; h < GM; ++h) {
+    qv[h] = h < G && on ? ikv::scale4(scale_log2, *reinterpret_cast<const float4 *>(s_q + h * 4 * LPK + 4 * c)) : zero;
+    o[h] = zero;
+    m[h] = -INFINITY;
+    l[h] = 0.f;
+  }
+  for (int j0 = t_begin + state; j0 - state < t_end; j0 += STATES * U) {
+    if (j0 - state != t_begin) load(j0);
+    if (newest) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + STATES * u == n_kv - 1 && on) {
+          kr[u] = *reinterpret_cast<const float4 *>(s_kn + 4 * c);
+          vr[u] = *reinterpret_cast<const float4 *>(s_vn + 4 * c);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < GM; ++h) {
+      if (h < G) {
+        float sc[U], mx = m[h];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float d = ikv::dot4(qv[h], kr[u]);
+          const float w = LPK == 16   ? ikv::row16_sum(d)
+                          : LPK == 32 ? ikv::half_wave_sum_valu(d)
+                                      : ikv::wave_sum(d);
+          sc[u] = j0 + STATES * u < t_end ? w : -INFINITY;
+          mx = fmaxf(mx, sc[u]);
+        }
+        // a lane group without a key yet keeps a zero state (reference 0)
+        const float ref = mx == -INFINITY ? 0.f : mx;
+        const float alpha = ikv::fast_exp2(m[h] - ref);
+        float psum = 0.f;
+        o[h] = ikv::scale4(alpha, o[h]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float pu = ikv::fast_exp2(sc[u] - ref);
+          psum += pu;
+          o[h] = ikv::fma4(pu, vr[u], o[h]);
+        }
+        l[h] = fmaf(l[h], alpha, psum);
+        m[h] = mx;
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < GM; ++h) {
+    if (h < G) {
+      if (c == 0) {
+        s_m[state][h] = m[h];
+        s_l[state][h] = l[h];
+      }
+      *reinterpret_cast<float4 *>(&s_o[state][h][4 * c]) = o[h];
+    }
+  }
+  __syncthreads();
+  const size_t rec0 = static_cast<size_t>(g) * G * n_splits + split;  // record of head 0
+  for (int idx = threadIdx.x; idx < G * dim; idx += 256) {
+    const int h = idx / dim, d = idx - h * dim;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < STATES; ++w) M = fmaxf(M, s_m[w][h]);
+    float L = 0.f, O = 0.f;
+#pragma unroll
+    for (int w = 0; w < STATES; ++w) {
+      const float mw = s_m[w][h];
+      const float e = mw == -INFINITY ? 0.f : ikv::fast_exp2(mw - M);
+      L = fmaf(e, s_l[w][h], L);
+      O = fmaf(e, s_o[w][h][d], O);
+    }
+    const size_t rec = rec0 + static_cast<size_t>(h) * n_splits;
+    part_o[rec * dim + d] = O;
+    if (d == 0) {
+      part_ml[2 * rec] = M;
+      part_ml[2 * rec + 1] = L;
+    }
   }
 }
 
@@ -474,6 +707,62 @@ size_t generic_decode_ws_bytes(int n_head, int n_head_kv, int head_dim, int64_t 
   if (!generic_attn_shape(n_head, n_head_kv, head_dim)) return 0;
   const SplitPlan p = split_plan(n_head, n_head_kv, head_dim, n_kv);
   return p.dl ? split_ws_bytes(n_head, head_dim, p.n_splits) : 0;
+}
+
+bool generic_decode_folds(const float *q, const float *k, const float *v, const float *k_new,
+                          const float *v_new, const Pages *pages, int n_head, int n_head_kv,
+                          int head_dim, int64_t n_kv, const void *workspace,
+                          size_t workspace_bytes, const DecodeNew *pro) {
+  if (head_dim % 4 != 0 || head_dim > 256 || n_head / n_head_kv > 8 || n_kv <= 0) return false;
+  if (!aligned16(k) || !aligned16(v) || !workspace || !aligned16(workspace)) return false;
+  const SplitPlan p = split_plan(n_head, n_head_kv, head_dim, n_kv);
+  if (!p.dl || workspace_bytes < split_ws_bytes(n_head, head_dim, p.n_splits)) return false;
+  if (pages && k_new && (!aligned16(v_new) || (!pro && !aligned16(k_new)))) return false;
+  if (!pro) return true;
+  // head_rope_kernel's head sizes and alignment: the same rows, bit for bit
+  if (head_dim != 64 && head_dim != 128 && head_dim != 256) return false;
+  for (const void *x : {static_cast<const void *>(q), static_cast<const void *>(k_new),
+                        static_cast<const void *>(pro->q_norm_w), static_cast<const void *>(pro->k_norm_w),
+                        static_cast<const void *>(pro->sin_tab), static_cast<const void *>(pro->cos_tab)})
+    if (reinterpret_cast<uintptr_t>(x) & 7) return false;
+  return true;
+}
+
+int attn_generic_decode_folded(const float *q, float *k, float *v, const float *k_new,
+                               const float *v_new, const Pages *pages, float *out, int n_head,
+                               int n_head_kv, int head_dim, int64_t n_kv, float scale,
+                               void *workspace, const DecodeNew *pro, hipStream_t s) {
+  const SplitPlan p = split_plan(n_head, n_head_kv, head_dim, n_kv);
+  if (!(scale > 0.0f)) scale = 1.0f / sqrtf(static_cast<float>(head_dim));
+  float *part_ml = static_cast<float *>(workspace);
+  float *part_o = part_ml + ((sizeof(float) * 2 * static_cast<size_t>(n_head) * p.n_splits + 255) & ~size_t(255)) / sizeof(float);
+  const unsigned grid = static_cast<unsigned>(n_head_kv) * static_cast<unsigned>(p.n_splits);
+  const int G = n_head / n_head_kv;
+  const Pages pg = pages ? *pages : Pages{};
+  const DecodeNew nw = pro ? *pro : DecodeNew{};
+#define IKV_ROWS(LPK, GM, PRO)                                                                        \
+  decode_rows_kernel<LPK, GM, PRO><<<grid, 256, 0, s>>>(                                              \
+      q, k, v, k_new, v_new, part_ml, part_o, n_head_kv, G, head_dim, static_cast<int>(n_kv),         \
+      p.keys_per_split, p.n_splits, scale * kLog2e, pages != nullptr, pg, nw)
+#define IKV_ROWS_G(LPK)                                                            \
+  do {                                                                             \
+    if (pro) {                                                                     \
+      if (G <= 4) IKV_ROWS(LPK, 4, true); else IKV_ROWS(LPK, 8, true);             \
+    } else {                                                                       \
+      if (G <= 4) IKV_ROWS(LPK, 4, false); else IKV_ROWS(LPK, 8, false);           \
+    }                                                                              \
+  } while (0)
+  if (head_dim <= 64)
+    IKV_ROWS_G(16);
+  else if (head_dim <= 128)
+    IKV_ROWS_G(32);
+  else
+    IKV_ROWS_G(64);
+#undef IKV_ROWS_G
+#undef IKV_ROWS
+  generic_merge_kernel<<<static_cast<unsigned>(n_head), kMergeThreads, 0, s>>>(part_ml, part_o, out,
+                                                                               head_dim, p.n_splits);
+  return launch_status();
 }
 
 int attn_generic_decode(const float *q, const float *k, const float *v, const Pages *pages,

@@ -38,4 +38,30 @@ int attn_generic_decode(const float *q, const float *k, const float *v, const Pa
                         float *out, int n_head, int n_head_kv, int head_dim, int64_t n_kv,
                         float scale, void *workspace, size_t workspace_bytes, hipStream_t s);
 
+// The qk-RMSNorm + RoPE of a decode step's new token (raw q and k rows in).
+struct DecodeNew {
+  const float *q_norm_w = nullptr, *k_norm_w = nullptr;
+  float eps = 0.f;
+  const int32_t *pos = nullptr;  // pos[0]: the new token's position
+  const float *sin_tab = nullptr, *cos_tab = nullptr;
+  int64_t n_ctx = 0;
+  int *status = nullptr;
+};
+
+// Whether attn_generic_decode_folded takes the step: rows of 16-byte pieces
+// (head_dim a multiple of 4 up to 256, aligned caches), at most 8 query heads
+// per KV head, room for the partials and, with pro, head_dim 64, 128 or 256 and
+// 8-byte aligned rows and tables. The new rows of a paged cache are 16-byte
+// aligned, as the append kernel asks.
+bool generic_decode_folds(const float *q, const float *k, const float *v, const float *k_new,
+                          const float *v_new, const Pages *pages, int n_head, int n_head_kv,
+                          int head_dim, int64_t n_kv, const void *workspace,
+                          size_t workspace_bytes, const DecodeNew *pro);
+// The step in two launches: [qk-norm + RoPE of q and k_new,] the append of
+// k_new and v_new (or NULL) at row n_kv - 1, the split attention; the merge.
+int attn_generic_decode_folded(const float *q, float *k, float *v, const float *k_new,
+                               const float *v_new, const Pages *pages, float *out, int n_head,
+                               int n_head_kv, int head_dim, int64_t n_kv, float scale,
+                               void *workspace, const DecodeNew *pro, hipStream_t s);
+
 }  // namespace ikv

@@ -37,6 +37,15 @@ constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // lane i <-> 7-i within 8 lanes
 constexpr int kDppMirror = 0x140;     // lane i <-> 15-i within 16 lanes
 
+// Sum over each 16 lanes, every lane getting it.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp<kDppXor1>(v);
+  v += dpp<kDppXor2>(v);
+  v += dpp<kDppHalfMirror>(v);
+  v += dpp<kDppMirror>(v);
+  return v;
+}
+
 // Sum over the 32 lanes of a half-wave; every lane of the half gets the sum.
 // Four DPP steps build sums over 4, 8 and 16 lanes; one ds_swizzle (xor 16
 // inside each 32-lane group, bitmask mode) finishes.
