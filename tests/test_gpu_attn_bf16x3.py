@@ -60,7 +60,10 @@ def test_against_64_bits(dev, n, past, H, KV, D):
 
 
 @pytest.mark.parametrize("n,past,H,KV,D,block", [(300, 700, 16, 8, 128, 64), (700, 900, 32, 8, 128, 256),
-                                                 (150, 333, 12, 4, 64, 64), (2100, 0, 12, 4, 64, 128)])
+                                                 (150, 333, 12, 4, 64, 64), (2100, 0, 12, 4, 64, 128),
+                                                 # more than 64 blocks
+                                                 (300, 8200, 16, 8, 128, 64), (777, 3500, 32, 8, 128, 64),
+                                                 (150, 4300, 12, 4, 64, 64), (2100, 2200, 12, 4, 64, 64)])
 def test_paged_equals_contiguous(dev, n, past, H, KV, D, block):
     rows = n + past
     q, k, v = (dev_t(70 + i + n, s, dev) for i, s in enumerate(((n, H, D), (rows, KV, D), (rows, KV, D))))
