@@ -249,10 +249,14 @@ def _ptr(t) -> Optional[int]:
 
 
 def _stream(stream=None) -> int:
+    if stream is not None:
+        return stream.cuda_stream
     torch = _torch()
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return stream.cuda_stream
+    if torch.cuda.is_initialized():
+        # the current stream's handle without a Stream object around it: 0.3 us
+        # against 2.9, of a call's 7.4 (a one-row norm)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _need_f32_dev(name: str, t) -> None:
