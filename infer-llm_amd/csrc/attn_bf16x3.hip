@@ -489,9 +489,10 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   if (kg != 0) return;
   float inv = 1.0f / pair_sum(l_part);
   // Inputs the pieces do not carry (bf16x3.hpp) leave a result that is not
-  // finite, or only tiny ones: the wave then starts over on F32 MFMAs, over
-  // the tiles its own rows see (a masked key weighs 0, and 0 times an infinite
-  // value is NaN: no row meets keys past its wave's last tile)
+  // finite, or only tiny ones: the wave then starts over, on F32 MFMAs over
+  // the tiles that all its rows see whole and key by key over the rest, where
+  // a row takes only the keys it sees (a masked key weighs 0, but 0 times an
+  // infinite value is NaN)
   bool odd = !(fabsf(inv) < INFINITY);
   float top = 0.f;
 #pragma unroll
@@ -510,8 +511,9 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
     l_part = 0.f;
     const float *qr = q + (static_cast<size_t>(tok) * n_head + head) * dim;
     const int last_tok = min(row0 + 31, n_rows - 1) / G;
-    const int my_tiles = (min(n_kv, n_past + last_tok + 1) + BN - 1) / BN;
-    for (int tile = 0; tile < my_tiles; ++tile) {
+    const int my_end = min(n_kv, n_past + last_tok + 1);
+    const int full = min(n_kv, n_past + first_tok + 1) / BN;  // tiles that every row sees whole
+    for (int tile = 0; tile < full; ++tile) {
       int first = tile * BN;
       if constexpr (PAGED) first += static_cast<int>(ikv::page_shift(pages, first));
       const auto rk = tile_rsrc(k, tile, first);
@@ -528,8 +530,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
       float p[16], mt = -INFINITY;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int kk = tile * BN + 8 * (e >> 2) + 4 * c2 + (e & 3);
-        p[e] = kk > n_past + tok || kk >= n_kv ? -INFINITY : s[e] * scale_log2;
+        p[e] = s[e] * scale_log2;
         mt = fmaxf(mt, p[e]);
       }
       const float m_new = fmaxf(m_row, pair_max(mt));
@@ -537,8 +538,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
       const float alpha = m_new == -INFINITY ? 1.f : ikv::fast_exp2(m_row - m_new);
       m_row = m_new;
       l_part *= alpha;
-#pragma unroll
-      for (int t = 0; t < DT; ++t) o[t] *= alpha;
+      floatx16 ot[DT] = {};  // this tile's sums
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const float x = ikv::fast_exp2(p[e] - ref);
@@ -548,9 +548,45 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
         for (int t = 0; t < DT; ++t) {
           const unsigned at = 32 * t + r32 < dim ? static_cast<unsigned>((key * stride + 32 * t + r32) * 4)
                                                  : 0x80000000u;
-          o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, at, 0, 0)), x, o[t], 0, 0, 0);
+          ot[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, at, 0, 0)), x, ot[t], 0, 0, 0);
         }
+      }
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[t] = o[t] * alpha + ot[t];
+    }
+    for (int key = full * BN; key < my_end; ++key) {
+      const bool sees = key <= n_past + tok;
+      int at = key;
+      if constexpr (PAGED) at += static_cast<int>(ikv::page_shift(pages, key));
+      const float *kr = k + static_cast<size_t>(at) * stride + g * dim;
+      const float *vr = v + static_cast<size_t>(at) * stride + g * dim;
+      float dot = 0.f;  // a lane's half of the dims
+      for (int d = 4 * c2; d < dim; d += 8) {
+        const floatx4 a = *reinterpret_cast<const floatx4 *>(kr + d);
+        const floatx4 b = *reinterpret_cast<const floatx4 *>(qr + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dot = fmaf(a[e], b[e], dot);
+      }
+      const float sc = pair_sum(dot) * scale_log2;
+      if (sees) {
+        const float m_new = fmaxf(m_row, sc);
+        const float ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = m_new == -INFINITY ? 1.f : ikv::fast_exp2(m_row - m_new);
+        const float x = ikv::fast_exp2(sc - ref);
+        m_row = m_new;
+        l_part = fmaf(l_part, alpha, c2 == 0 ? x : 0.f);
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int z = 0; z < 4; ++z) {
+            const int d = 32 * t + 8 * z + 4 * c2;
+            if (d < dim) {
+              const floatx4 y = *reinterpret_cast<const floatx4 *>(vr + d);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[t][4 * z + e] = fmaf(x, y[e], o[t][4 * z + e] * alpha);
+            }
+          }
       }
     }
     inv = 1.0f / pair_sum(l_part);
@@ -626,6 +662,9 @@ int attn_bf16x3(const float *q, const float *k, const float *v, const Pages *pag
   if (!(scale > 0.0f)) scale = 1.0f / sqrtf(static_cast<float>(head_dim));
   const float sl2 = scale * kLog2e;
   const int64_t rows = n_q * G;
+  // cache rows behind the prompt (a longer cache, its rows not yet written)
+  // are not read: a masked key's weight of 0 would not silence a NaN there
+  n_kv = std::min(n_kv, n_past + n_q);
   auto steps = [&](int br, int kg, int slots) {
     return steps_of(rows, G, n_kv, n_past, n_head_kv, br, kg, slots);
   };

@@ -86,8 +86,6 @@ def test_values_the_pieces_cannot_carry(dev, n, H, KV, D):
     q[:, :, 0] = q[:, :, 0].abs() + 0.5
     base = attn64(q, k, v, 0)
     # an infinite value reaches the rows that see its key, in its own dim only
-    # (key 192 opens a tile and its rows a wave: a masked key's weight of zero
-    # times infinity is NaN within those)
     v2 = v.clone()
     v2[192, 1, 3] = float("inf")
     got = ikv.attn_prefill(q, k, v2, 0)
@@ -120,3 +118,42 @@ def test_values_the_pieces_cannot_carry(dev, n, H, KV, D):
     for ex in (-100, -120):
         got = ikv.attn_prefill(q, k, v * 2.0 ** ex, 0)
         assert float((got.double() * 2.0 ** -ex - base).norm() / base.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("n,past,H,KV,D", [
+    (100, 0, 12, 4, 64), (1000, 17, 12, 4, 64), (2501, 0, 12, 4, 64), (150, 3, 10, 5, 80),
+    (300, 5, 16, 8, 128), (2050, 0, 32, 8, 128), (1, 99, 10, 5, 80)])
+def test_rows_behind_the_prompt_are_not_read(dev, n, past, H, KV, D):
+    # a longer cache whose later rows hold no numbers: in the last tile of
+    # keys, and past it
+    q, k, v = (dev_t(110 + i + n, s, dev) for i, s in
+               enumerate(((n, H, D), (n + past, KV, D), (n + past, KV, D))))
+    want = ikv.attn_prefill(q, k, v, past)
+    block = 64
+    rows = -(-(n + past + 150) // block) * block
+    for what in ("nan", "inf"):
+        caches = []
+        for t in (k, v):
+            caches.append(torch.full((rows, KV, D), float(what), device=dev))
+            caches[-1][:n + past] = t
+        assert torch.equal(ikv.attn_prefill(q, *caches, past, n_kv=rows), want)
+        table = torch.arange(rows // block, dtype=torch.int32, device=dev)
+        assert torch.equal(ikv.attn_prefill_paged(q, *caches, table, block, past, n_kv=rows), want)
+
+
+@pytest.mark.parametrize("n,H,KV,D", [(400, 16, 8, 128), (2300, 32, 8, 128), (400, 12, 4, 64), (2500, 12, 4, 64)])
+@pytest.mark.parametrize("key", [0, 203, 319])
+def test_a_value_that_is_no_number_reaches_no_earlier_row(dev, n, H, KV, D, key):
+    q, k, v = (dev_t(120 + i, s, dev) for i, s in enumerate(((n, H, D), (n, KV, D), (n, KV, D))))
+    base = attn64(q, k, v, 0)
+    G = H // KV
+    for bad in (float("inf"), float("nan")):
+        v2 = v.clone()
+        v2[key, 1, 3] = bad
+        got = ikv.attn_prefill(q, k, v2, 0)
+        hit = torch.zeros_like(base, dtype=torch.bool)
+        hit[key:, G:2 * G, 3] = True
+        assert bool((got[hit].isnan() if bad != bad else got[hit] == bad).all())
+        assert bool(((got.double() - base).abs() <= 1e-5 + 1e-4 * base.abs())[~hit].all())
+        # the wave that starts over sums in another order, not with fewer bits
+        assert float((got.double() - base)[~hit].norm() / base[~hit].norm()) <= 2 ** -23 * (8 + math.sqrt(n))
