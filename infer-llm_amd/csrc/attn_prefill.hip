@@ -561,6 +561,9 @@ int prefill_common(const float *q, const float *k, const float *v, const ikv_kv_
   if (n_head_kv > kMaxKvHeads) return -EOVERFLOW;
   if (!ikv::aligned16(q) || !ikv::aligned16(k) || !ikv::aligned16(v) || !ikv::aligned16(out))
     return -EINVAL;
+  // cache rows behind the prompt (a longer cache, its rows not yet written)
+  // are staged as zeros: a masked key's weight of 0 would not silence a NaN
+  n_kv = std::min(n_kv, n_past + n_q);
   if (!(scale > 0.0f)) scale = 1.0f / sqrtf(static_cast<float>(head_dim));
   const float sl2 = scale * ikv::kLog2e;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -571,7 +574,7 @@ int prefill_common(const float *q, const float *k, const float *v, const ikv_kv_
   // against 21.5); past both, 300 tokens 26.4 against 24.1 us, 2048 150
   // against 122.
   const int64_t row_blocks = (n_q * G + 15) / 16;
-  if (row_blocks * n_head_kv > kCUs && std::min(n_kv, n_past + n_q) > 256 &&
+  if (row_blocks * n_head_kv > kCUs && n_kv > 256 &&
       ikv::attn_bf16x3_supported(q, k, v, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past))
     return ikv::attn_bf16x3(q, k, v, pg, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past, scale, s);
   const int nq = static_cast<int>(n_q), nk = static_cast<int>(n_kv), np = static_cast<int>(n_past);

@@ -122,7 +122,9 @@ def test_values_the_pieces_cannot_carry(dev, n, H, KV, D):
 
 @pytest.mark.parametrize("n,past,H,KV,D", [
     (100, 0, 12, 4, 64), (1000, 17, 12, 4, 64), (2501, 0, 12, 4, 64), (150, 3, 10, 5, 80),
-    (300, 5, 16, 8, 128), (2050, 0, 32, 8, 128), (1, 99, 10, 5, 80)])
+    (300, 5, 16, 8, 128), (2050, 0, 32, 8, 128), (1, 99, 10, 5, 80),
+    # prompts of the F32 MFMA kernel, in one, two and four wave groups
+    (1, 0, 16, 8, 128), (37, 0, 16, 8, 128), (77, 1000, 16, 8, 128), (200, 3, 32, 8, 128), (600, 0, 8, 1, 128)])
 def test_rows_behind_the_prompt_are_not_read(dev, n, past, H, KV, D):
     # a longer cache whose later rows hold no numbers: in the last tile of
     # keys, and past it
