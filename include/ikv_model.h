@@ -34,7 +34,8 @@ extern "C" {
  * ikv_gemm_nt_f32 or, for products large enough, the same product on bf16
  * MFMA with every float split into three exact bf16 pieces (F32 inputs,
  * sums and results; no farther from a 64-bit product than the F32 MFMA
- * kernel), with K split over several workgroups when the tiles
+ * kernel: an output tile whose operands hold an infinity, a NaN or bits below
+ * bf16's smallest, 2^-133, is formed on F32 MFMA), with K split over several workgroups when the tiles
  * would leave compute units idle: such a call needs a split-K workspace of
  * its device and stream, which the first one allocates (8 MiB + 16 KiB,
  * kept until exit; so make it outside HIP graph capture; -ENOMEM after 64

@@ -62,6 +62,8 @@ using namespace ikv::pieces;
 constexpr int kCUs = 256;         // MI355X compute units
 constexpr int BN = 32;            // keys per tile
 constexpr float kRescale = 8.0f;  // log2 headroom before the running max is moved
+// Results that are all below this may come from inputs below 2^-109.
+constexpr float kTinySum = 0x1p-64f;
 
 __device__ __forceinline__ float pair_max(float x) {  // lanes l and l ^ 32
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -132,6 +134,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   unsigned short *const sk = s_k[kg];
   floatx4 kraw[VD][2];
   float vraw[8][VD];
+  unsigned lost = 0;
   // (first: the tile's row of the cache or the pool)
   auto tile_rsrc = [&](const float *base, int tile, int first) {
     const int rows = min(BN, n_kv - tile * BN);
@@ -155,7 +158,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   auto put_k = [&]() {
 #pragma unroll
     for (int i = 0; i < VD; ++i) {
-      const Pieces p = split8(kraw[i][0], kraw[i][1]);
+      const Pieces p = split8(kraw[i][0], kraw[i][1], lost);
 #pragma unroll
       for (int z = 0; z < 3; ++z) *reinterpret_cast<bf16x8 *>(sk + z * PLANE + kdst[i]) = p.p[z];
     }
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
 #pragma unroll
     for (int i = 0; i < VD; ++i) {
       const Pieces p = split8(floatx4{vraw[0][i], vraw[1][i], vraw[2][i], vraw[3][i]},
-                              floatx4{vraw[4][i], vraw[5][i], vraw[6][i], vraw[7][i]});
+                              floatx4{vraw[4][i], vraw[5][i], vraw[6][i], vraw[7][i]}, lost);
 #pragma unroll
       for (int z = 0; z < 3; ++z) *reinterpret_cast<bf16x8 *>(sv + z * PLANE + v_at(vd0 + i, vc)) = p.p[z];
     }
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
       floatx4 u{}, w{};
       if (row_ok && d < dim) u = *reinterpret_cast<const floatx4 *>(qr + d);
       if (row_ok && d + 4 < dim) w = *reinterpret_cast<const floatx4 *>(qr + d + 4);
-      const Pieces p = split8(u, w);
+      const Pieces p = split8(u, w, lost);
 #pragma unroll
       for (int z = 0; z < 3; ++z) qp[s][z] = p.p[z];
     }
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
 #pragma unroll
           for (int e = 2 * h; e < 2 * h + 2; ++e) {
             unsigned x, y, z;
-            split2(p[8 * t + 2 * e], p[8 * t + 2 * e + 1], x, y, z);
+            split2(p[8 * t + 2 * e], p[8 * t + 2 * e + 1], x, y, z, lost);
             asm volatile("" : "+v"(x), "+v"(y), "+v"(z));
             pw[t][0][e] = x, pw[t][1][e] = y, pw[t][2][e] = z;
           }
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           unsigned y0, y1, y2;
-          split2(x[2 * e], x[2 * e + 1], y0, y1, y2);
+          split2(x[2 * e], x[2 * e + 1], y0, y1, y2, lost);
           // (pinned to this region: the first half has no use in it)
           asm volatile("" : "+v"(y0), "+v"(y1), "+v"(y2));
           cw[0][2 * h + e] = y0, cw[1][2 * h + e] = y1, cw[2][2 * h + e] = y2;

@@ -19,7 +19,12 @@
 // groups or splits (their partial sums are smaller); gemm_plan takes it only
 // where the F32 kernel's plan has no more K ranges than this one's.
 //
-// Inputs that the split does not carry are caught at the end (see kTinySum).
+// Inputs that the split does not carry are found as they are split, or by the
+// sums they leave, and the tile is formed again on F32 MFMAs. Looking at every
+// split costs 0.6% of 4096-token products and 1-3% of those that the VALU
+// bounds (4096 x 4096 at 509 tokens 99.5 -> 101.7 us); one look at the largest
+// sum of a wave cost nothing, and missed a small row among ordinary ones and
+// small floats against large ones.
 //
 // Layout:
 //   * A workgroup owns BW weight rows x BT tokens: WM wavefronts (per K
@@ -30,7 +35,7 @@
 //     are split once per workgroup and staged in LDS as three bf16 planes.
 //     That halves the LDS traffic of staging both (a product reads 12 bytes
 //     of pieces per 8 of F32).
-//   * 32 x 32 x 16 rather than 16 x 16 x 32: a wave issues the 44 VALU
+//   * 32 x 32 x 16 rather than 16 x 16 x 32: a wave issues the 48 VALU
 //     instructions of 8 floats' split between MFMAs, and four of them behind
 //     one 32-cycle MFMA cost half a cycle (probe: 16.5 cycles per half MFMA),
 //     while two behind a 16-cycle one cost 4.5.
@@ -85,6 +90,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   constexpr int LDS_HALFS = KG * 2 * 3 * PLANE;
   constexpr int XCH_HALFS = (KG - 1) * TM * TN * WM * 64 * 16 * 2;
   __shared__ int s_last;
+  __shared__ int s_lost;
   __shared__ __attribute__((aligned(16))) unsigned short s_x[LDS_HALFS > XCH_HALFS ? LDS_HALFS : XCH_HALFS];
 
   const int b = static_cast<int>(blockIdx.x);
@@ -149,6 +155,8 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   floatx4 wr[2 * TM][2], xr[NX][2];  // step s + 1's floats, then step s + 2's
   Pieces a[2][TM][2];
   bf16x8 bc[2][3];
+  unsigned lost = 0;  // what this thread's splits dropped
+  if (threadIdx.x == 0) s_lost = 0;
 
   auto load_w = [&](int u, int st) {
     const int off = (k_lo + min(st, n_steps - 1) * BK) * 4;
@@ -162,7 +170,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   };
   unsigned short *const sx = s_x + kg * (2 * 3 * PLANE);
   auto put_x = [&](int i, unsigned short *buf) {
-    const Pieces s = split8(xr[i][0], xr[i][1]);
+    const Pieces s = split8(xr[i][0], xr[i][1], lost);
 #pragma unroll
     for (int p = 0; p < 3; ++p)
       *reinterpret_cast<bf16x8 *>(buf + p * PLANE + xdst[i]) = s.p[p];
@@ -198,7 +206,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
           load_x(u, s + 2);
         } else {
           const int v = u - NX;
-          a[P ^ 1][v / 2][v & 1] = split8(wr[v][0], wr[v][1]);
+          a[P ^ 1][v / 2][v & 1] = split8(wr[v][0], wr[v][1], lost);
           load_w(v, s + 2);
         }
       }
@@ -239,7 +247,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   }
 #pragma unroll
   for (int i = 0; i < 2 * TM; ++i) {
-    a[0][i / 2][i & 1] = split8(wr[i][0], wr[i][1]);
+    a[0][i / 2][i & 1] = split8(wr[i][0], wr[i][1], lost);
     load_w(i, 1);
   }
   __syncthreads();
@@ -256,14 +264,19 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   }
   if (s < n_steps) step(s, P0{});
 
+  // (a token's pieces serve every wave: if any split dropped bits, all start
+  // over)
+  if (any_lost(lost) && lane == 0) s_lost = 1;
+  __syncthreads();
+  const bool redo = s_lost != 0;
+
   auto quad = [&](int i, int j, int q) {
     return floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                    acc[i][j][4 * q + 3]};
   };
   const bool mine = KG == 1 || kg == 0;  // group 0 ends with the tile's sums
   if constexpr (KG > 1) {
-    floatx4 *const xch = reinterpret_cast<floatx4 *>(s_x);
-    __syncthreads();
+    floatx4 *const xch = reinterpret_cast<floatx4 *>(s_x);  // (its readers are past the barrier above)
     if (!mine) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -291,48 +304,42 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   }
 
   // Inputs the split does not carry: an infinite or NaN input (or one that
-  // rounds to an infinite bf16) leaves NaNs in the sums, and pieces of inputs
-  // below 2^-109 fall off bf16's range, which matters only if every sum is
-  // tiny. Such a wave redoes its sums with F32 MFMAs from memory.
+  // rounds to an infinite bf16) leaves NaNs in the wave's sums, and splits of
+  // floats below 2^-109 may have dropped bits. The sums are then formed again
+  // with F32 MFMAs from memory, 128 columns at a time.
   if (mine) {
-    bool odd = false;
-    float top = 0.f;
+    bool odd = redo;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float v = fabsf(acc[i][j][r]);
-          odd |= !(v < INFINITY);
-          top = fmaxf(top, v);
-        }
-    top = ikv::wave_max(top);
-    if (__builtin_amdgcn_ballot_w64(odd) != 0 || (top > 0.f && top < kTinySum)) {
+        for (int r = 0; r < 16; ++r) odd |= !(fabsf(acc[i][j][r]) < INFINITY);
+    if (__builtin_amdgcn_ballot_w64(odd) != 0) {
+      // (an MFMA tile at a time: this path is to cost the main loop no registers)
+      const int kb1 = s_hi * KG * BK;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
-      const int kb0 = s_lo * KG * BK, kb1 = s_hi * KG * BK;
-      // MFMA e of 8 columns from kb contracts columns kb + e and kb + 4 + e
-      for (int kb = kb0; kb < kb1; kb += 8) {
-        floatx4 av[TM], bv[TN];
+        for (int j = 0; j < TN; ++j) {
+          const unsigned wo = static_cast<unsigned>((((wave * TM + i) * 32 + r32) * k + 4 * c2) * 4);
+          const unsigned xo = static_cast<unsigned>(((32 * j + r32) * k + 4 * c2) * 4);
+          acc[i][j] = floatx16{};
+#pragma unroll 1
+          for (int kb0 = s_lo * KG * BK; kb0 < kb1; kb0 += 128) {
+            floatx16 sum{};
+            // MFMA e of 8 columns from kb contracts columns kb + e and kb + 4 + e
+#pragma unroll 1
+            for (int kb = kb0; kb < min(kb0 + 128, kb1); kb += 8) {
+              const floatx4 av = __builtin_amdgcn_raw_buffer_load_b128(rw, wo, kb * 4, 0);
+              const floatx4 bv = __builtin_amdgcn_raw_buffer_load_b128(rx, xo, kb * 4, 0);
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-          av[i] = __builtin_amdgcn_raw_buffer_load_b128(
-              rw, static_cast<unsigned>((((wave * TM + i) * 32 + r32) * k + 4 * c2) * 4), kb * 4, 0);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          bv[j] = __builtin_amdgcn_raw_buffer_load_b128(
-              rx, static_cast<unsigned>(((32 * j + r32) * k + 4 * c2) * 4), kb * 4, 0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
-      }
+              for (int e = 0; e < 4; ++e)
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[e], sum, 0, 0, 0);
+            }
+            acc[i][j] += sum;
+          }
+        }
     }
   }
 

@@ -102,3 +102,40 @@ def test_the_plan_takes_it_for_large_products(dev, n_out, k, m):
     assert code.value in PIECE_TILES
     w, x = dev_t(40, (n_out, k), 0.02, dev), dev_t(41, (m, k), 1.0, dev)
     assert torch.equal(ikv.mul_mat(w, x), tile(code.value, split.value, w, x))
+
+
+@pytest.mark.parametrize("code", PIECE_TILES)
+@pytest.mark.parametrize("split", [1, 2])
+def test_small_floats_keep_their_bits_beside_ordinary_ones(dev, code, split):
+    # a float below 2^-109 has bits that no bf16 piece holds: one such token
+    # among ordinary ones, one such weight row, one such element in a row, and
+    # whole operands of them against large ones. Row by row and column by
+    # column no farther from 64 bits than the F32 kernel's sums can be:
+    # 2^-24 sqrt(k) of |x| |w|, and what a denormal result rounds by
+    n_out, k, m = 256, 256, 128
+    w0, x0 = dev_t(50, (n_out, k), 0.02, dev), dev_t(51, (m, k), 1.0, dev)
+
+    def check(x, w, what):
+        got = tile(code, split, w, x).double()
+        xd, wd = x.double(), w.double()
+        bar = 2.0 ** -24 * k ** 0.5 * xd.norm(dim=1)[:, None] * wd.norm(dim=1)[None] + k * 2.0 ** -149
+        assert bool(((got - xd @ wd.t()).abs() <= bar).all()), what
+
+    for ex in (-109, -112, -115, -122, -126, -132, -140):
+        x, w = x0.clone(), w0.clone()
+        x[77] *= 2.0 ** ex
+        check(x, w0, ("token", ex))
+        w[200] *= 2.0 ** (ex + 6)
+        check(x0, w, ("weight row", ex))
+        # (the row's other products are zero)
+        x = x0.clone()
+        x[5] = 0
+        x[5, 200] = 1.2345678 * 2.0 ** ex
+        check(x, w0 * 2.0 ** 60, ("element", ex))
+        x, w = x0 * 2.0 ** ex, w0 * 2.0 ** min(100, -ex - 30)
+        check(x, w, ("against large", ex))
+        check(w[:m] * 1.0, (x0 * 2.0 ** ex).repeat(2, 1), ("large against", ex))
+    # products that are denormal or next to it, of floats that are not
+    x, w = x0.clone(), w0 * 2.0 ** -60
+    x[::3] *= 2.0 ** -60
+    check(x, w, "denormal sums")
