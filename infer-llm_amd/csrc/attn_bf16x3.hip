@@ -43,6 +43,14 @@
 //     TFLOP/s), 777 behind 3319 467 -> 290; 0.6B heads, 2048 tokens 150 ->
 //     122; 12 heads of 64 over 4, 1500 behind 500 232 -> 68; 12 of 128 over 4,
 //     512 tokens 59 -> 35.
+//   * What the pieces do not carry: a wave starts over on F32 where its sums
+//     are not finite, or where a split of V or Q dropped bits (floats below
+//     2^-109; V's are looked at one by one, as a dim of small values has only
+//     small sums) or Q is so large that bits dropped from K would count;
+//     probabilities are split times 2^17. That costs 1-3% (0.6B heads, 2048
+//     tokens 112.7 -> 115.7 us cold); one look at a wave's largest output cost
+//     nothing, and missed a small dim among ordinary ones and small keys
+//     against large queries.
 //   * Tried and not kept: two waves per SIMD with Q's last pieces in LDS (0.6B
 //     2048 125, 8B 4096 824: 256 registers leave no room to schedule in); K
 //     and V two tiles ahead (equal); blocks in pairs of a long and a short one
@@ -62,8 +70,10 @@ using namespace ikv::pieces;
 constexpr int kCUs = 256;         // MI355X compute units
 constexpr int BN = 32;            // keys per tile
 constexpr float kRescale = 8.0f;  // log2 headroom before the running max is moved
-// Results that are all below this may come from inputs below 2^-109.
-constexpr float kTinySum = 0x1p-64f;
+// Probabilities go into their pieces (and the row sums) times 2^17, so that all
+// down to the smallest normal float, which is as small as exp2 gives them, keep
+// their bits. The factor leaves with the division by the row's sum.
+constexpr float kProbScale = 0x1p17f;
 
 __device__ __forceinline__ float pair_max(float x) {  // lanes l and l ^ 32
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -134,7 +144,9 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   unsigned short *const sk = s_k[kg];
   floatx4 kraw[VD][2];
   float vraw[8][VD];
-  unsigned lost = 0;
+  unsigned lost = 0;  // what this thread's splits of Q and V dropped
+  __shared__ int s_lost;
+  if (threadIdx.x == 0) s_lost = 0;
   // (first: the tile's row of the cache or the pool)
   auto tile_rsrc = [&](const float *base, int tile, int first) {
     const int rows = min(BN, n_kv - tile * BN);
@@ -158,7 +170,8 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   auto put_k = [&]() {
 #pragma unroll
     for (int i = 0; i < VD; ++i) {
-      const Pieces p = split8(kraw[i][0], kraw[i][1], lost);
+      unsigned none = 0;
+      const Pieces p = split8<false>(kraw[i][0], kraw[i][1], none);
 #pragma unroll
       for (int z = 0; z < 3; ++z) *reinterpret_cast<bf16x8 *>(sk + z * PLANE + kdst[i]) = p.p[z];
     }
@@ -166,7 +179,7 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   auto put_v = [&](unsigned short *sv) {
 #pragma unroll
     for (int i = 0; i < VD; ++i) {
-      const Pieces p = split8(floatx4{vraw[0][i], vraw[1][i], vraw[2][i], vraw[3][i]},
+      const Pieces p = split8<false>(floatx4{vraw[0][i], vraw[1][i], vraw[2][i], vraw[3][i]},
                               floatx4{vraw[4][i], vraw[5][i], vraw[6][i], vraw[7][i]}, lost);
 #pragma unroll
       for (int z = 0; z < 3; ++z) *reinterpret_cast<bf16x8 *>(sv + z * PLANE + v_at(vd0 + i, vc)) = p.p[z];
@@ -235,16 +248,22 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   bf16x8 qp[KS][3];
   {
     const float *qr = q + (static_cast<size_t>(tok) * n_head + head) * dim;
+    float top = 0.f;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const int d = 16 * s + 8 * c2;
       floatx4 u{}, w{};
       if (row_ok && d < dim) u = *reinterpret_cast<const floatx4 *>(qr + d);
       if (row_ok && d + 4 < dim) w = *reinterpret_cast<const floatx4 *>(qr + d + 4);
-      const Pieces p = split8(u, w, lost);
+      const Pieces p = split8<false>(u, w, lost);
 #pragma unroll
       for (int z = 0; z < 3; ++z) qp[s][z] = p.p[z];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) top = fmaxf(fmaxf(top, fabsf(u[e])), fabsf(w[e]));
     }
+    // Bits dropped from K (below 2^-133) move a score by less than 2^-60 times
+    // this bound on Q: K's splits are not looked at.
+    if (top * fmaxf(scale_log2, 1.f) >= 0x1p64f) lost = ~0u;
   }
   floatx16 o[DT];
 #pragma unroll
@@ -325,15 +344,15 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
         if constexpr (w % 3 == 0) {
 #pragma unroll
           for (int e = 8 * t; e < 8 * t + 8; ++e) {
-            p[e] = ikv::fast_exp2(fmaf(p[e], scale_log2, -ref));
+            p[e] = ikv::fast_exp2(fmaf(p[e], scale_log2, -ref)) * kProbScale;
             l_part += p[e];
           }
         } else {
           constexpr int h = w % 3 - 1;
 #pragma unroll
           for (int e = 2 * h; e < 2 * h + 2; ++e) {
-            unsigned x, y, z;
-            split2(p[8 * t + 2 * e], p[8 * t + 2 * e + 1], x, y, z, lost);
+            unsigned x, y, z, none = 0;
+            split2(p[8 * t + 2 * e], p[8 * t + 2 * e + 1], x, y, z, none);
             asm volatile("" : "+v"(x), "+v"(y), "+v"(z));
             pw[t][0][e] = x, pw[t][1][e] = y, pw[t][2][e] = z;
           }
@@ -341,12 +360,13 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
       });
       if constexpr (s == 1) load_v(staged(i + 1), row_1);
       qk(s);
+      constexpr int kShare = s == 0 ? 3 : 4 * (hi - lo) + 2 * ((hi + 2) / 3 - (lo + 2) / 3);  // 8 of exp are 32
 #pragma unroll
       for (int z = 0; z < 6; ++z) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         if (s == 1 && z > 0) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
         if (z % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, s == 0 ? 3 : 4 * (hi - lo), 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, kShare, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (s == 0) {
@@ -375,17 +395,19 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
       static_for<hi - lo>([&](auto wc) {
         constexpr int w = lo + decltype(wc)::value, u = w / 2, h = w & 1;
         float x[4];
+        unsigned none = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           x[e] = u < VD ? kraw[u % VD][h][e] : vraw[4 * h + e][u % VD];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           unsigned y0, y1, y2;
-          split2(x[2 * e], x[2 * e + 1], y0, y1, y2, lost);
+          split2(x[2 * e], x[2 * e + 1], y0, y1, y2, u < VD ? none : lost);
           // (pinned to this region: the first half has no use in it)
           asm volatile("" : "+v"(y0), "+v"(y1), "+v"(y2));
           cw[0][2 * h + e] = y0, cw[1][2 * h + e] = y1, cw[2][2 * h + e] = y2;
         }
+        if constexpr (u >= VD) asm volatile("" : "+v"(lost));
         if constexpr (h == 1) {
           unsigned short *dst = u < VD ? sk + kdst[u % VD] : s_v[kg][P ^ 1] + v_at(vd0 + u % VD, vc);
 #pragma unroll
@@ -457,6 +479,8 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
     }
   }
 
+  if (any_lost(lost) && lane == 0) s_lost = 1;  // (V's pieces serve every wave)
+  if constexpr (KG == 1) __syncthreads();
   if constexpr (KG > 1) {
     // the groups' states meet in LDS: groups 1 .. hand theirs to group 0
     constexpr int XW = 16 * DT + 2;
@@ -491,23 +515,17 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
   }
   if (kg != 0) return;
   float inv = 1.0f / pair_sum(l_part);
-  // Inputs the pieces do not carry (bf16x3.hpp) leave a result that is not
-  // finite, or only tiny ones: the wave then starts over, on F32 MFMAs over
+  // Inputs the pieces do not carry (bf16x3.hpp) dropped bits in a split or leave
+  // a result that is not finite: the wave then starts over, on F32 MFMAs over
   // the tiles that all its rows see whole and key by key over the rest, where
   // a row takes only the keys it sees (a masked key weighs 0, but 0 times an
   // infinite value is NaN)
-  bool odd = !(fabsf(inv) < INFINITY);
-  float top = 0.f;
+  bool odd = s_lost != 0 || !(fabsf(inv) < INFINITY);
 #pragma unroll
   for (int t = 0; t < DT; ++t)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float x = fabsf(o[t][e] * inv);
-      odd |= !(x < INFINITY);
-      top = fmaxf(top, x);
-    }
-  top = ikv::wave_max(top);
-  if (__builtin_amdgcn_ballot_w64(odd) != 0 || (top > 0.f && top < kTinySum)) {
+    for (int e = 0; e < 16; ++e) odd |= !(fabsf(o[t][e] * inv) < INFINITY);
+  if (__builtin_amdgcn_ballot_w64(odd) != 0) {
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = floatx16{};
     m_row = -INFINITY;

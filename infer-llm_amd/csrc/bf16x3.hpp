@@ -46,6 +46,11 @@ __device__ __forceinline__ void split2(float a, float b, unsigned &h, unsigned &
   l = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
   lost |= __float_as_uint(sa) | __float_as_uint(sb);
 }
+// PIN: what is dropped is collected with the last piece, so that the third
+// residues need no registers past it (GEMM loops; one chain through `lost` for
+// all splits was 2% slower there, and straight-line code schedules better
+// without).
+template <bool PIN>
 __device__ __forceinline__ Pieces split8(floatx4 u, floatx4 v, unsigned &lost) {
   uintx4 q[3];
   unsigned t = 0;
@@ -61,9 +66,7 @@ __device__ __forceinline__ Pieces split8(floatx4 u, floatx4 v, unsigned &lost) {
     q[2][e] = l;
   }
   lost |= t;
-  // (t is formed with the last piece, and the third residues need no registers
-  // past it; one chain through `lost` for all splits was 2% slower)
-  asm("" : "+v"(q[2][3]), "+v"(lost));
+  if constexpr (PIN) asm("" : "+v"(q[2][3]), "+v"(lost));
   return Pieces{{__builtin_bit_cast(bf16x8, q[0]), __builtin_bit_cast(bf16x8, q[1]),
                  __builtin_bit_cast(bf16x8, q[2])}};
 }

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   };
   unsigned short *const sx = s_x + kg * (2 * 3 * PLANE);
   auto put_x = [&](int i, unsigned short *buf) {
-    const Pieces s = split8(xr[i][0], xr[i][1], lost);
+    const Pieces s = split8<true>(xr[i][0], xr[i][1], lost);
 #pragma unroll
     for (int p = 0; p < 3; ++p)
       *reinterpret_cast<bf16x8 *>(buf + p * PLANE + xdst[i]) = s.p[p];
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
           load_x(u, s + 2);
         } else {
           const int v = u - NX;
-          a[P ^ 1][v / 2][v & 1] = split8(wr[v][0], wr[v][1], lost);
+          a[P ^ 1][v / 2][v & 1] = split8<true>(wr[v][0], wr[v][1], lost);
           load_w(v, s + 2);
         }
       }
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(WM * KG * 64, MINW) void gemm_bf16x3_kernel(
   }
 #pragma unroll
   for (int i = 0; i < 2 * TM; ++i) {
-    a[0][i / 2][i & 1] = split8(wr[i][0], wr[i][1], lost);
+    a[0][i / 2][i & 1] = split8<true>(wr[i][0], wr[i][1], lost);
     load_w(i, 1);
   }
   __syncthreads();

@@ -159,3 +159,52 @@ def test_a_value_that_is_no_number_reaches_no_earlier_row(dev, n, H, KV, D, key)
         assert bool(((got.double() - base).abs() <= 1e-5 + 1e-4 * base.abs())[~hit].all())
         # the wave that starts over sums in another order, not with fewer bits
         assert float((got.double() - base)[~hit].norm() / base[~hit].norm()) <= 2 ** -23 * (8 + math.sqrt(n))
+
+
+@pytest.mark.parametrize("n,past,H,KV,D", [(400, 0, 16, 8, 128), (2300, 0, 32, 8, 128), (400, 7, 12, 4, 64),
+                                           (2500, 0, 12, 4, 64)])
+def test_small_floats_keep_their_bits_beside_ordinary_ones(dev, n, past, H, KV, D):
+    # a float below 2^-109 has bits that no bf16 piece holds: dims, keys and
+    # whole values of them, queries of them against large keys and keys of them
+    # against large queries. Dim by dim and head by head as far from 64 bits as
+    # F32 sums are
+    q, k, v = (dev_t(130 + i, s, dev) for i, s in
+               enumerate(((n, H, D), (n + past, KV, D), (n + past, KV, D))))
+    bar = 2 ** -23 * (8 + math.sqrt(n + past))
+
+    def check(q, k, v, what, bar=bar):
+        got, ref = ikv.attn_prefill(q, k, v, past).double(), attn64(q, k, v, past)
+        floor = n * 2.0 ** -149  # of denormal results
+        assert bool(((got - ref).norm(dim=0) <= bar * ref.norm(dim=0) + floor).all()), what
+
+    for ex in (-109, -115, -122, -128):
+        v2 = v.clone()
+        v2[:, :, 5] *= 2.0 ** ex
+        check(q, k, v2, ("dim", ex))
+        check(q, k, v * 2.0 ** ex, ("values", ex))
+        check(q * 2.0 ** ex, k * 2.0 ** min(-ex, 120), v, ("queries", ex))
+        k2, q2 = k.clone(), q.clone()
+        k2[:, :, 7] *= 2.0 ** ex
+        q2[:, :, 7] *= 2.0 ** min(-ex, 120)
+        check(q2, k2, v, ("keys", ex))
+
+
+@pytest.mark.parametrize("n,H,KV,D", [(400, 16, 8, 128), (2300, 32, 8, 128), (400, 12, 4, 64), (2500, 12, 4, 64)])
+@pytest.mark.parametrize("nats", [70, 80, 86])
+def test_small_probabilities_keep_their_bits(dev, n, H, KV, D, nats):
+    # key 0 takes nearly all the weight and its value is zero: a row is the sum
+    # of the others' weights near e^-nats (2^-101, 2^-115, 2^-124)
+    q, k, v = (dev_t(140 + i, s, dev) for i, s in enumerate(((n, H, D), (n, KV, D), (n, KV, D))))
+    q *= 0.1
+    q[:, :, 0] = math.sqrt(D)
+    k[:, :, 0] = -float(nats)
+    k[0] = 0
+    v = v.abs()
+    v[0] = 0
+    got, ref = ikv.attn_prefill(q, k, v, 0).double(), attn64(q, k, v, 0)
+    # a score of this size is rounded to 2^-24 of it at each of its sum's D / 16
+    # matrix steps (the first dim puts it there), where the two parts of the sum
+    # meet, at its scale and at its distance from the largest; pieces that
+    # drop bits below 2^-133 are off by 2^-9 at 86
+    bar = (D / 16 + 3) * nats * 2 ** -24 + 2 ** -23 * (8 + math.sqrt(n))
+    assert bool(((got - ref).norm(dim=2) <= bar * ref.norm(dim=2)).all())
