@@ -35,13 +35,15 @@ extern "C" {
  * MFMA with every float split into three exact bf16 pieces (F32 inputs,
  * sums and results; no farther from a 64-bit product than the F32 MFMA
  * kernel: an output tile whose operands hold an infinity, a NaN or bits below
- * bf16's smallest, 2^-133, is formed on F32 MFMA), with K split over several workgroups when the tiles
- * would leave compute units idle: such a call needs a split-K workspace of
- * its device and stream, which the first one allocates (8 MiB + 16 KiB,
- * kept until exit; so make it outside HIP graph capture; -ENOMEM after 64
- * device-stream pairs). Any other shape runs one wavefront per output
- * (m <= 65535, else -ENOTSUP). Every path is deterministic: a fixed
- * summation order per output for given n_out, k and m.
+ * bf16's smallest, 2^-133, is formed on F32 MFMA), with K split over several
+ * workgroups when the tiles would leave compute units idle: such a call needs
+ * a split-K workspace of its device and stream, which the first one allocates
+ * (8 MiB + 16 KiB, kept until exit; so make it outside HIP graph capture;
+ * -ENOMEM after 64 device-stream pairs). A product that only the bf16 plan
+ * splits does without where none can be had, its sums then in the unsplit
+ * order. Any other shape runs one wavefront per output (m <= 65535, else
+ * -ENOTSUP). Every path is deterministic: a fixed summation order per output
+ * for given n_out, k and m.
  * residual: NULL, or [m][n_out] added to the result (out may equal
  * residual).
  * ------------------------------------------------------------------- */

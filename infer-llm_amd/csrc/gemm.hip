@@ -495,7 +495,8 @@ __global__ void zero_ints_kernel(int *p, int n) {
 // The split-K workspace of (current device, stream s): allocated and its
 // counters cleared (a kernel on s) on the first call for the pair, kept
 // until the process ends. Calls on one stream are ordered, so they never
-// share a workspace at the same time.
+// share a workspace at the same time. Nothing is allocated while s is captured
+// (hipErrorStreamCaptureUnsupported, and the capture goes on).
 int split_workspace(hipStream_t s, float **part, int **counters) {
   struct Entry {
     int dev;
@@ -517,6 +518,11 @@ int split_workspace(hipStream_t s, float **part, int **counters) {
       return 0;
     }
   if (n_entries == kMaxEntries) return -ENOMEM;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  e = hipStreamIsCapturing(s, &capturing);
+  if (e != hipSuccess) return static_cast<int>(e);
+  if (capturing != hipStreamCaptureStatusNone)
+    return static_cast<int>(hipErrorStreamCaptureUnsupported);
   void *mem = nullptr;
   e = hipMalloc(&mem, kSplitCounterBytes + kSplitPartBytes);
   if (e != hipSuccess) return static_cast<int>(e);
@@ -621,12 +627,16 @@ int gemm_nt_f32(const float *w, const float *x, float *out, const float *residua
                 int64_t k, int64_t m, bool may_split, hipStream_t s) {
   if (!gemm_nt_supported(n_out, k, m)) return -ENOTSUP;
   if (!aligned16(w) || !aligned16(x)) return -EINVAL;
-  const GemmPlan p = gemm_plan(n_out, k, m, may_split);
+  GemmPlan p = gemm_plan(n_out, k, m, may_split);
   float *part = nullptr;
   int *counters = nullptr;
   if (p.split > 1) {
     const int rc = split_workspace(s, &part, &counters);
-    if (rc) return rc;
+    if (rc) {
+      // the F32 kernel's plan asks for no workspace here: nor does the product
+      if (gemm_f32_plan(n_out, k, m, may_split, nullptr).split > 1) return rc;
+      p = gemm_plan(n_out, k, m, false);
+    }
   }
   return gemm_nt_tile(p.tile, p.split, w, x, out, residual, static_cast<int>(n_out),
                       static_cast<int>(k), static_cast<int>(m), part, counters, s);

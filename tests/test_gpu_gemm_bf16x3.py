@@ -139,3 +139,48 @@ def test_small_floats_keep_their_bits_beside_ordinary_ones(dev, code, split):
     x, w = x0.clone(), w0 * 2.0 ** -60
     x[::3] *= 2.0 ** -60
     check(x, w, "denormal sums")
+
+
+def test_a_split_the_f32_plan_does_not_ask_for_needs_no_workspace(dev):
+    # captured on a stream that never ran such a product, so without a
+    # workspace: the product runs unsplit, as it did on the F32 kernel; one
+    # that the F32 plan splits as well is refused, and the capture goes on
+    lib = ikv.load_bench()
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def plan(name, n_out, k, m):
+        code, split = ctypes.c_int(), ctypes.c_int()
+        assert getattr(lib, name)(n_out, k, m, ctypes.byref(code), ctypes.byref(split)) == 0
+        return code.value, split.value
+
+    n_out, k, m = 4096, 4096, 128
+    assert plan("ikv_bench_gemm_plan", n_out, k, m)[1] == 1
+    assert plan("ikv_bench_gemm_choice", n_out, k, m)[1] > 1
+    assert plan("ikv_bench_gemm_plan", 1024, 2048, 128)[1] > 1
+    w, x = dev_t(60, (n_out, k), 0.02, dev), dev_t(61, (m, k), 1.0, dev)
+    w2, x2 = dev_t(62, (1024, 2048), 0.02, dev), dev_t(63, (128, 2048), 1.0, dev)
+    out, out2 = torch.empty(m, n_out, device=dev), torch.zeros(128, 1024, device=dev)
+    eager = ikv.mul_mat(w, x)
+    raw = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(raw)) == 0
+    side = torch.cuda.ExternalStream(raw.value)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        ikv.mul_mat(w, x, out=out)
+        with pytest.raises(RuntimeError):
+            ikv.mul_mat(w2, x2, out=out2)
+        ikv.mul_mat(w, x, out=out)
+    scale = x.double().norm(dim=1)[:, None] * w.double().norm(dim=1)[None]
+    ref = x.double() @ w.double().t()
+    first = None
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert bool(((out.double() - ref).abs() <= 2.0 ** -24 * k ** 0.5 * scale).all())
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first)
+    assert rel(eager, ref) <= rel(out, ref) * 1.5 and not out2.any()
+    del g
+    assert hip.hipStreamDestroy(raw) == 0
