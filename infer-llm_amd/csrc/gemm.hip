@@ -443,19 +443,25 @@ constexpr int kNumTiles = 5;
 // split + per_split * (S - 1) for S > 1), us[q - 1] the time of a 64-column
 // step of q workgroups on a CU. Fitted (non-negative least squares, 5-8% rms)
 // to 12 projection shapes (n_out 256-12288, k 768-12288) at ten token counts
-// from 72 to 4096, every split; the F32 model's units are 0.24 us there, plus
-// 4.2 us. Over that sweep the plan is on average 0.7% slower than the best
-// choice and 1.18 times as fast as the F32 kernel alone.
+// from 72 to 4096, every split; then 0.6 us and 3% added for the look at what
+// the splits drop. The F32 kernel, for the choice between the two: kF32Us, by
+// the same fit over 476 products with k from 64. Over those (n_out 128-12288,
+// k 64-12288, 65-4096 tokens) the plan is on average 0.7% slower than the best
+// choice, 1.13 times as fast as the F32 kernel alone and nowhere more than 3%
+// slower than it; before short sums were in the fit, a k of 64 ran 1.4 times
+// and k of 128-640 1.1-1.2 times as long as on the F32 kernel (8192 x 64 at 65
+// tokens 6.4 us against 5.1, 512 x 512 at 1100 10.9 against 9.9).
 struct Bf16x3Shape {
   int bt, bw, groups, res;  // tokens, weight rows, K groups, workgroups per CU
   double fixed, us[3], split, per_split;
 };
-constexpr Bf16x3Shape kBf16x3[] = {{128, 256, 1, 1, 9.3, {3.0, 0, 0}, 3.2, 8.2},
-                                   {128, 128, 1, 2, 5.7, {1.74, 4.11, 0}, 2.7, 4.1},
-                                   {64, 128, 1, 3, 4.1, {1.2, 2.47, 4.18}, 2.0, 2.2},
-                                   {64, 64, 2, 3, 4.6, {0.73, 1.38, 2.29}, 1.3, 2.2}};
+constexpr Bf16x3Shape kBf16x3[] = {{128, 256, 1, 1, 9.9, {3.09, 0, 0}, 3.3, 8.45},
+                                   {128, 128, 1, 2, 6.3, {1.79, 4.23, 0}, 2.8, 4.2},
+                                   {64, 128, 1, 3, 4.7, {1.24, 2.54, 4.31}, 2.1, 2.3},
+                                   {64, 64, 2, 3, 5.2, {0.75, 1.42, 2.36}, 1.3, 2.3}};
 constexpr int kNumBf16x3 = 4;
-constexpr double kUnitUs = 0.24, kFixedUs = 4.2;
+// fixed, per round and step of the tile's cost, per round of it, for a split
+constexpr double kF32Us[] = {2.85, 0.258, 0.505, 1.74};
 constexpr double kBf16x3Margin = 0.95;  // taken when it promises 5% over the F32 kernel
 constexpr double kFillSteps = 2.0;
 constexpr int kMinSplitSteps = 4;   // steps of BK columns per split, at least
@@ -548,7 +554,7 @@ bool gemm_nt_supported(int64_t n_out, int64_t k, int64_t m) {
          k <= kMaxK && m <= INT_MAX / 2;
 }
 
-GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, double *units) {
+GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, double *us) {
   const int n = static_cast<int>(n_out), mm = static_cast<int>(m);
   const int steps = static_cast<int>(k / BK);
   // the least estimated time; on a tie the larger tile, then fewer splits
@@ -568,13 +574,18 @@ GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, doub
       }
     }
   }
-  if (units) *units = best;
+  if (us) {
+    const double rounds = double((tile_count(p.tile, n, mm) * p.split + kCUs - 1) / kCUs);
+    const double cost = rounds * kTiles[p.tile].cost;
+    *us = kF32Us[0] + kF32Us[1] * cost * steps / p.split + kF32Us[2] * cost +
+          (p.split > 1 ? kF32Us[3] : 0.0);
+  }
   return p;
 }
 
 GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split) {
-  double best;
-  GemmPlan p = gemm_f32_plan(n_out, k, m, may_split, &best);
+  double f32_us;
+  GemmPlan p = gemm_f32_plan(n_out, k, m, may_split, &f32_us);
   if (!gemm_bf16x3_supported(n_out, k, m)) return p;
   const int n = static_cast<int>(n_out), mm = static_cast<int>(m);
   const int steps = static_cast<int>(k / BK);
@@ -582,7 +593,7 @@ GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split) {
   // many K ranges as the F32 plan (each halving of a sum's length takes about
   // 1.4 off its rounding error, and the pieces start 1.15 ahead)
   const int f32_split = p.split;
-  double best_us = kBf16x3Margin * (kFixedUs + kUnitUs * best);
+  double best_us = kBf16x3Margin * f32_us;
   for (int i = 0; i < kNumBf16x3; ++i) {
     const Bf16x3Shape &t = kBf16x3[i];
     const int64_t tiles = tile_count(t, n, mm);

@@ -19,9 +19,9 @@ struct GemmPlan {
   int tile;
   int split;
 };
-// The F32 MFMA kernel's plan and its estimate in the cost model's units, and
-// the choice between it and the bf16-piece kernel.
-GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, double *units);
+// The F32 MFMA kernel's plan and its estimated time, and the choice between it
+// and the bf16-piece kernel.
+GemmPlan gemm_f32_plan(int64_t n_out, int64_t k, int64_t m, bool may_split, double *us);
 GemmPlan gemm_plan(int64_t n_out, int64_t k, int64_t m, bool may_split);
 
 // One launch on tile shape `tile` (tokens x outputs; F32 MFMA: 0 128 x 128

@@ -80,6 +80,33 @@ def test_gemm_plan(n_out, k, m, plan):
     assert f"{GEMM_TILE_NAMES[tile.value]}/{split.value}" == plan
 
 
+PIECE_TILE_NAMES = ["128x256", "128x128", "64x128", "64x64"]  # tile codes from 5
+
+
+@pytest.mark.parametrize("n_out,k,m,plan", [
+    # short sums: a piece kernel's start and end are not worth it
+    (256, 64, 1100, "f32 64x32/1"), (8192, 64, 65, "f32 32x32/1"), (2048, 256, 333, "f32 32x32/1"),
+    (512, 512, 1100, "f32 32x32/1"), (8192, 640, 65, "f32 32x32/1"),
+    # a round of 32x32 tiles, where the 64x64 pieces would leave CUs idle
+    (2048, 1024, 333, "f32 32x32/1"), (3072, 1024, 200, "f32 32x32/1"),
+    (1024, 4096, 128, "f32 32x32/2"), (64, 4096, 300, "f32 32x32/8"),
+    # and past it
+    (2048, 1024, 509, "pieces 64x64/1"), (1024, 768, 916, "pieces 64x64/1"),
+    (4096, 4096, 128, "pieces 64x64/2"), (1024, 3072, 777, "pieces 64x128/2"),
+    (12288, 4096, 65, "f32 32x32/1"), (12288, 4096, 128, "pieces 64x128/1"),
+    (2048, 1024, 2048, "pieces 128x128/1"), (8192, 64, 4096, "pieces 128x256/1"),
+    (4096, 12288, 4096, "pieces 128x256/1"),
+])
+def test_gemm_choice(n_out, k, m, plan):
+    import ctypes
+    tile, split = ctypes.c_int(), ctypes.c_int()
+    assert ikv.load_bench().ikv_bench_gemm_choice(n_out, k, m, ctypes.byref(tile),
+                                                  ctypes.byref(split)) == 0
+    name = (f"f32 {GEMM_TILE_NAMES[tile.value]}" if tile.value < 5
+            else f"pieces {PIECE_TILE_NAMES[tile.value - 5]}")
+    assert f"{name}/{split.value}" == plan
+
+
 def test_library_does_not_link_the_oracle():
     deps = subprocess.run(["ldd", str(ikv.LIB_PATH)], capture_output=True, text=True).stdout
     assert "oracle" not in deps
