@@ -263,10 +263,14 @@ __global__ __launch_bounds__(kThreads) void gemv_swiglu_kernel(const float *__re
 // columns of 1024 rows are 3 MB): the pieces of 1024 columns, of the row and of
 // x, load together, where gemv_generic_kernel asks for four bytes a lane and
 // waits for them every few steps. A piece past the row loads the row's last one
-// and counts as zeros, so that no branch stands between the loads.
+// and counts as zeros, so that no branch stands between the loads; U of them, as
+// many as a row of up to 1024 columns has per lane (with four, a row of 256
+// loaded its last piece three times: 12288 rows 6.15 us against 3.6 of
+// gemv_generic_kernel).
 // Graphs of 20 launches over weights of their own, before and now: 1024 rows of
 // 768 5.6 -> 3.0 us, 3072 of 2304 19.3 -> 8.3, 1000 of 3076 16.4 -> 5.1; 64
 // tokens of 1000 x 1000 39.9 -> 24.5.
+template <int U>
 __global__ __launch_bounds__(kThreads) void gemv_pieces_kernel(const float *__restrict__ w,
                                                                const float *__restrict__ x, float *out,
                                                                const float *residual, int n_out, int K) {
@@ -277,7 +281,6 @@ __global__ __launch_bounds__(kThreads) void gemv_pieces_kernel(const float *__re
   const float4 *row = reinterpret_cast<const float4 *>(w + static_cast<size_t>(n) * K);
   const float4 *xt = reinterpret_cast<const float4 *>(x + token * K);
   const int n4 = K / 4;
-  constexpr int U = 4;
   float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int c0 = lane; c0 - lane < n4; c0 += 64 * U) {
     float4 wv[U], xv[U];
@@ -494,6 +497,10 @@ bool skinny_ok(int64_t n_out, int64_t k, int64_t m, std::initializer_list<const 
 
 }  // namespace
 
+// Outputs of a product of several tokens from which rows of 257 to 383 floats
+// take the generic kernel: eight waves on every SIMD.
+constexpr int64_t kShortTurnOutputs = 8192;
+
 extern "C" int ikv_mul_mat_f32(const float *w, const float *x, float *out, int64_t n_out,
                                int64_t k, int64_t m, const float *residual, void *stream) {
   if (!w || !x || !out) return -EINVAL;
@@ -504,13 +511,20 @@ extern "C" int ikv_mul_mat_f32(const float *w, const float *x, float *out, int64
   hipStream_t s = static_cast<hipStream_t>(stream);
   // a wave per output: for rows of 16-byte pieces, and for any (fewer than 64
   // pieces leave lanes idle: 64 columns 2.35 us against 2.23, 260 2.53 against
-  // 2.90)
+  // 2.90; so does a second turn for less than 32 where tokens share the weights
+  // in L2: 60 rows of 260 at 300 tokens 5.9 us against 4.6)
   auto launch_any = [&](unsigned tokens) {
     const dim3 grid(grid_for(n_out), tokens);
-    if (k >= 256 && k % 4 == 0 && ikv::aligned16(w) && ikv::aligned16(x))
-      gemv_pieces_kernel<<<grid, kThreads, 0, s>>>(w, x, out, residual, int(n_out), int(k));
-    else
+    const bool short_turn = tokens > 1 && k > 256 && k < 384 && n_out * tokens >= kShortTurnOutputs;
+    if (k >= 256 && !short_turn && k % 4 == 0 && ikv::aligned16(w) && ikv::aligned16(x)) {
+      const auto kernel = k <= 256   ? gemv_pieces_kernel<1>
+                          : k <= 512 ? gemv_pieces_kernel<2>
+                          : k <= 768 ? gemv_pieces_kernel<3>
+                                     : gemv_pieces_kernel<4>;
+      kernel<<<grid, kThreads, 0, s>>>(w, x, out, residual, int(n_out), int(k));
+    } else {
       gemv_generic_kernel<<<grid, kThreads, 0, s>>>(w, x, out, residual, int(n_out), int(k), 0, nullptr);
+    }
   };
   if (m == 1) {
     if (fast_ok(k, {w, x})) {

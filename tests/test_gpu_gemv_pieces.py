@@ -10,8 +10,8 @@ from ikv import synth
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("k", [1, 4, 7, 252, 256, 260, 768, 1020, 1028, 2044, 3076])
-@pytest.mark.parametrize("n_out,m", [(1, 1), (5, 1), (1024, 1), (67, 3)])
+@pytest.mark.parametrize("k", [1, 4, 7, 252, 256, 260, 380, 384, 512, 516, 768, 1020, 1028, 2044, 3076])
+@pytest.mark.parametrize("n_out,m", [(1, 1), (5, 1), (1024, 1), (67, 3), (300, 28)])
 def test_rows(dev, k, n_out, m):
     # one piece up to several rounds of 1024 columns, remainders in each; an
     # output is a sum of k products, 2^-24 (k + 1) of the sum of their sizes
