@@ -256,7 +256,9 @@ __global__ __launch_bounds__(kRowThreads) void row_kernel(const float *__restric
 // 256 * NV floats are loaded once, all loads in flight together, and stay in
 // registers (NV = 0: longer rows, read twice). Graphs of 20 launches: 4096 rows
 // of 4096 floats 292 us (mostly one wave's index-order sum) -> 22.5 (5.9 TB/s),
-// 1024 rows 9.7 -> 7.3, one row 5.0 -> 3.5; 2048 rows of 1024 4.5 -> 4.2.
+// 1024 rows 9.7 -> 7.3, one row 5.0 -> 3.5; 2048 rows of 1024 4.5 -> 4.2. Five
+// sizes of NV, since the pieces past a row cost: 2048 rows of 1280 5.85 us with
+// 16 of them, 4.44 with 6 (4.7 read twice); 4096 of 2560 15.7 and, with 12, 13.8.
 template <int NV>
 __global__ __launch_bounds__(256) void long_row_norm_kernel(const float *__restrict__ x,
                                                             const float *__restrict__ w, float *out,
@@ -477,6 +479,9 @@ extern "C" int ikv_rms_norm_f32(const float *x, const float *w, float *out, int6
     const int64_t blocks = (rows + 3) / 4;
     if (blocks > INT_MAX) return -EOVERFLOW;
     const auto kernel = dim <= 1024   ? long_row_norm_kernel<4>
+                        : dim <= 1536 ? long_row_norm_kernel<6>
+                        : dim <= 2048 ? long_row_norm_kernel<8>
+                        : dim <= 3072 ? long_row_norm_kernel<12>
                         : dim <= 4096 ? long_row_norm_kernel<16>
                                       : long_row_norm_kernel<0>;
     kernel<<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(

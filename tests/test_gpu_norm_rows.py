@@ -45,7 +45,7 @@ def midpoint_rows(dim, n, seed):
     return x
 
 
-@pytest.mark.parametrize("dim", [256, 768, 1024, 1280, 4096, 8192])
+@pytest.mark.parametrize("dim", [256, 768, 1024, 1280, 1536, 1792, 2048, 2304, 3072, 3328, 4096, 8192])
 def test_midpoint_rows_long(dev, dim):
     x, w = midpoint_rows(dim, 9, 900 + dim), synth.normal(901, (dim,))
     got = ikv.rms_norm(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), float(EPS))
