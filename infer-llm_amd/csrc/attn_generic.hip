@@ -365,31 +365,39 @@ __global__ __launch_bounds__(kSplitWaves * 64) void generic_split_kernel(
 // one workgroup per query head. Wave 0 forms the weights (lanes over splits)
 // and the sum; the threads take output dims, and where a head has at most
 // 128 of them several threads share a dim, each taking a run of the splits,
-// the runs added in order. All latency: a thread's first kMergeAhead partials
-// load while wave 0 forms the weights (40 splits of 64 dims 4.1 -> 3.7 us).
+// the runs added in order. All latency: a thread's first AHEAD partials load
+// while wave 0 forms the weights (40 splits of 64 dims 4.1 -> 3.7 us), and no
+// branch stands between the loads or between the weights (with one per split, a
+// decode step of 6 heads of 300 over 2 at 9000 keys took 45 us, 35 without).
 constexpr int kMergeThreads = 256;
-constexpr int kMergeAhead = 16;
+constexpr int kMaxAhead = 16;
+constexpr int merge_runs(int dim) { return dim <= 64 ? 4 : dim <= 128 ? 2 : 1; }
+template <int AHEAD>
 __global__ __launch_bounds__(kMergeThreads) void generic_merge_kernel(
     const float *__restrict__ part_ml, const float *__restrict__ part_o, float *__restrict__ out,
     int dim, int n_splits) {
   constexpr int kPerLane = kSplitTargetWgs / 64;
-  __shared__ float s_e[kSplitTargetWgs];
+  __shared__ float s_e[kSplitTargetWgs + kMaxAhead];
   __shared__ float s_L;
   __shared__ float s_part[kMergeThreads];
   const int head = blockIdx.x;
   const size_t rec0 = static_cast<size_t>(head) * n_splits;
-  const int runs = dim <= 64 ? 4 : dim <= 128 ? 2 : 1;
+  const int runs = merge_runs(dim);
   const int per = kMergeThreads / runs, r = threadIdx.x / per;
   const int lo = r * n_splits / runs, hi = (r + 1) * n_splits / runs;
-  float a[kMergeAhead];
+  float a[AHEAD];
+  // no branch between the loads (past the run: the last split's, as 0)
   auto load = [&](int d, int sp0) {
 #pragma unroll
-    for (int u = 0; u < kMergeAhead; ++u) {
-      a[u] = 0.f;
-      if (d < dim && sp0 + u < hi) a[u] = part_o[(rec0 + sp0 + u) * dim + d];
-    }
+    for (int u = 0; u < AHEAD; ++u)
+      a[u] = part_o[(rec0 + min(sp0 + u, n_splits - 1)) * dim + min(d, dim - 1)];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (sp0 + u >= hi) a[u] = 0.f;
   };
   load(threadIdx.x % per, lo);
+  if (threadIdx.x >= kMergeThreads - kMaxAhead)
+    s_e[kSplitTargetWgs + kMergeThreads - 1 - threadIdx.x] = 0.f;
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     float2 ml[kPerLane];
@@ -416,11 +424,11 @@ __global__ __launch_bounds__(kMergeThreads) void generic_merge_kernel(
   const float inv = 1.0f / s_L;
   auto run = [&](int d) {
     float O = 0.f;
-    for (int sp = lo; sp < hi; sp += kMergeAhead) {
+    for (int sp = lo; sp < hi; sp += AHEAD) {
       if (sp != lo) load(d, sp);
+      // (a branch per split made each wait for its weight alone)
 #pragma unroll
-      for (int u = 0; u < kMergeAhead; ++u)
-        if (sp + u < hi) O = fmaf(s_e[sp + u], a[u], O);
+      for (int u = 0; u < AHEAD; ++u) O = fmaf(s_e[sp + u], a[u], O);
     }
     return O;
   };
@@ -439,6 +447,13 @@ __global__ __launch_bounds__(kMergeThreads) void generic_merge_kernel(
     if (d != static_cast<int>(threadIdx.x)) load(d, lo);
     out[static_cast<size_t>(head) * dim + d] = run(d) * inv;
   }
+}
+
+void merge(const float *part_ml, const float *part_o, float *out, int n_head, int dim, int n_splits,
+           hipStream_t s) {
+  // (few splits: a short batch, whose loads past the run cost less)
+  const auto kernel = n_splits <= 4 * merge_runs(dim) ? generic_merge_kernel<4> : generic_merge_kernel<kMaxAhead>;
+  kernel<<<static_cast<unsigned>(n_head), kMergeThreads, 0, s>>>(part_ml, part_o, out, dim, n_splits);
 }
 
 // The split decode for rows of 16-byte pieces: head_dim a multiple of 4 up to
@@ -760,8 +775,7 @@ int attn_generic_decode_folded(const float *q, float *k, float *v, const float *
     IKV_ROWS_G(64);
 #undef IKV_ROWS_G
 #undef IKV_ROWS
-  generic_merge_kernel<<<static_cast<unsigned>(n_head), kMergeThreads, 0, s>>>(part_ml, part_o, out,
-                                                                               head_dim, p.n_splits);
+  merge(part_ml, part_o, out, n_head, head_dim, p.n_splits, s);
   return launch_status();
 }
 
@@ -795,8 +809,7 @@ int attn_generic_decode(const float *q, const float *k, const float *v, const Pa
     default: IKV_GENERIC_SPLIT(8); break;
   }
 #undef IKV_GENERIC_SPLIT
-  generic_merge_kernel<<<static_cast<unsigned>(n_head), kMergeThreads, 0, s>>>(
-      part_ml, part_o, out, head_dim, p.n_splits);
+  merge(part_ml, part_o, out, n_head, head_dim, p.n_splits, s);
   return launch_status();
 }
 

@@ -47,7 +47,9 @@ def attend64(q, k, v):
 @pytest.mark.parametrize("D,Hq,Hkv,n_kv", [
     (4, 3, 1, 1), (20, 5, 5, 65), (60, 14, 2, 300), (64, 12, 4, 64), (64, 21, 3, 4100),
     (68, 6, 2, 63), (124, 15, 5, 129), (128, 6, 2, 1000), (132, 7, 1, 31), (256, 16, 2, 97),
-    (252, 10, 2, 2049), (64, 18, 2, 200)])  # the last: 9 query heads, not folded
+    (252, 10, 2, 2049), (64, 18, 2, 200),  # the last from here: not folded
+    # merges of 1, of 16 n and of 256 splits, dims past a workgroup's threads
+    (30, 6, 2, 3), (300, 3, 1, 2048), (300, 6, 2, 2100), (512, 2, 1, 16384), (96, 9, 1, 16400)])
 def test_rows_at_the_edges(dev, D, Hq, Hkv, n_kv):
     seed = 7100 + D + n_kv
     k, v = synth.normal(seed, (n_kv, Hkv, D)), synth.normal(seed + 1, (n_kv, Hkv, D))
