@@ -423,7 +423,9 @@ __global__ __launch_bounds__(RW * KG * 64, MINW) void attn_bf16x3_kernel(
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         if (j == DT && z > 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
         if (j + 2 < 2 * DT && z % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 4 * (hi - lo), 0);
+        // (one more where V's splits also collect what they drop: 2% of the
+        // forms of two groups)
+        __builtin_amdgcn_sched_group_barrier(0x002, 4 * (hi - lo) + (j >= DT ? 1 : 0), 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -644,21 +646,37 @@ void launch(const float *q, const float *k, const float *v, float *out, int n_he
 
 namespace {
 
-int tiles_of(int64_t row, int G, int64_t n_kv, int64_t n_past) {  // of a row's visible keys
-  return static_cast<int>((std::min(n_kv, n_past + row / G + 1) + BN - 1) / BN);
+// A form of the kernel and its estimated time: blocks of `rows` rows, `groups`
+// key groups, `slots` workgroups on the card at once. us = fixed + the larger
+// of alone * (the longest block's steps) and busy * (the busiest slot's: the
+// average per slot, plus a shortest block where they do not divide evenly; the
+// longest blocks start first), a step being a tile of each group and a block's
+// start and end counting as `ends` steps more. Fitted to 1110 prompts (3 to
+// 128 heads of 32 to 128 over 1 to 128, 65-4096 tokens behind 0-4000): 3-6%
+// rms, and the first form up to 64 dims 15% where it is not the better one; on
+// average 0.1% from the better form of two. Without the blocks' ends a card
+// full of short ones took the wrong one: 128 heads of 64, 140 tokens 27.8 us
+// against 12.3, 64 heads, 400 tokens 43.7 against 20.0.
+struct Form {
+  int rows, groups, slots;
+  double fixed, alone, busy, ends;
+};
+
+double time_of(const Form &f, int64_t rows, int G, int64_t n_kv, int64_t n_past, int heads) {
+  auto steps = [&](int64_t row) {  // of a block that ends with this row
+    const int64_t tiles = (std::min(n_kv, n_past + row / G + 1) + BN - 1) / BN;
+    return static_cast<double>((tiles + f.groups - 1) / f.groups) + f.ends;
+  };
+  const double first = steps(std::min<int64_t>(f.rows, rows) - 1), last = steps(rows - 1);
+  const double per_slot = double((rows + f.rows - 1) / f.rows) * heads / f.slots;
+  const double load = per_slot * (first + last) / 2 + (std::ceil(per_slot) - per_slot) * first;
+  return f.fixed + std::max(f.alone * last, f.busy * load);
 }
 
-// Estimated tile steps of the busiest workgroup slot: blocks of br rows, kg
-// key groups, the longest blocks started first. At least the longest block;
-// else the average per slot, plus a shortest block where the blocks do not
-// divide evenly.
-double steps_of(int64_t rows, int G, int64_t n_kv, int64_t n_past, int heads, int br, int kg, int slots) {
-  const int64_t n = (rows + br - 1) / br;
-  const double first = double(tiles_of(std::min<int64_t>(br, rows) - 1, G, n_kv, n_past)) / kg;
-  const double last = double(tiles_of(rows - 1, G, n_kv, n_past)) / kg;
-  const double per_slot = double(n) * heads / slots;
-  return std::max(last, per_slot * (first + last) / 2 + (std::ceil(per_slot) - per_slot) * first);
-}
+// heads of 128: 128 rows and one key group, or 64 and two; heads of 64: 64 rows
+// and two groups, two workgroups on a CU, or 32 rows and four groups
+constexpr Form kForms128[2] = {{128, 1, kCUs, 0.0, 2.37, 2.37, 3.3}, {64, 2, kCUs, 0.0, 2.8, 2.8, 3.4}};
+constexpr Form kForms64[2] = {{64, 2, 2 * kCUs, 0.0, 1.74, 1.91, 3.5}, {32, 4, kCUs, 1.6, 2.37, 2.37, 2.5}};
 
 }  // namespace
 
@@ -686,29 +704,17 @@ int attn_bf16x3(const float *q, const float *k, const float *v, const Pages *pag
   // cache rows behind the prompt (a longer cache, its rows not yet written)
   // are not read: a masked key's weight of 0 would not silence a NaN there
   n_kv = std::min(n_kv, n_past + n_q);
-  auto steps = [&](int br, int kg, int slots) {
-    return steps_of(rows, G, n_kv, n_past, n_head_kv, br, kg, slots);
-  };
+  auto us = [&](const Form &f) { return time_of(f, rows, G, n_kv, n_past, n_head_kv); };
 #define IKV_A3(...)                                                                                \
   launch<__VA_ARGS__>(q, k, v, out, n_head_kv, G, head_dim, static_cast<int>(rows),                \
                       static_cast<int>(n_kv), static_cast<int>(n_past), sl2, pages, s)
   if (head_dim > 64) {
-    // 128 rows and one key group where that keeps the CUs busy, else 64 rows
-    // and two: a step of the latter stages twice the tiles and takes 1.22
-    // times as long (Qwen3-8B heads, 4096 tokens: 682 us against 795; 0.6B
-    // heads, 2048 tokens: 155 against 122)
-    if (steps(128, 1, kCUs) <= 1.22 * steps(64, 2, kCUs))
+    if (us(kForms128[0]) <= us(kForms128[1]))
       IKV_A3(4, 4, 1, 1);
     else
       IKV_A3(4, 2, 2, 1);
   } else {
-    // 64 rows, two groups and two workgroups on a CU (1.9 us a step alone,
-    // 3.3 beside another), or 32 rows and four groups (2.4 us, 3.2 with every
-    // CU busy): 12 heads of 64 over 4, 3870 tokens 151 us against 239; 200
-    // tokens behind 2000 69 against 48
-    const double two = std::max(1.9 * steps(64, 2, INT_MAX), 3.3 * steps(64, 2, 2 * kCUs));
-    const double four = std::max(2.4 * steps(32, 4, INT_MAX), 3.2 * steps(32, 4, kCUs));
-    if (two <= four)
+    if (us(kForms64[0]) <= us(kForms64[1]))
       IKV_A3(2, 2, 2, 2);
     else
       IKV_A3(2, 1, 4, 1);

@@ -48,7 +48,8 @@ __device__ __forceinline__ int64_t key_row(const ikv::Pages &pg, bool paged, int
 // Keys of the longest row from which attn_bf16x3 takes a prompt: 12 heads of
 // 64 over 4, 64 tokens 7.4 us here against 8.3 there, 128 tokens 11.0 against
 // 10.5, 37 tokens behind 1000 65 against 28; heads of 80, 100 tokens 16.6
-// against 14.5.
+// against 14.5. From here on it was ahead at every shape measured (3 to 128
+// heads of 32 to 96 over 1 to 128, up to 3500 tokens).
 constexpr int64_t kPiecesMinKeys = 96;
 
 constexpr int kTileRowsPerWave = 4;  // 8 measured slower (fewer workgroups, more registers)

@@ -571,10 +571,10 @@ int prefill_common(const float *q, const float *k, const float *v, const ikv_kv_
   // kernel. Up to one block per CU this kernel's one-wave groups win (0.6B
   // heads, 256 tokens 11.4 us against 20.9, 64 tokens behind 1000 26 against
   // 53), and so do its larger blocks on short rows (64 heads, 200 tokens 19.1
-  // against 21.5); past both, 300 tokens 26.4 against 24.1 us, 2048 150
-  // against 122.
-  const int64_t row_blocks = (n_q * G + 15) / 16;
-  if (row_blocks * n_head_kv > kCUs && n_kv > 256 &&
+  // against 21.5, 64 over 64, 257 tokens 28.3 against 29.0); past both, 300
+  // tokens 26.4 against 24.1 us, 2048 150 against 122.
+  const int64_t blocks = (n_q * G + 15) / 16 * n_head_kv;
+  if (blocks > kCUs && n_kv > (blocks > 4 * kCUs ? 288 : 256) &&
       ikv::attn_bf16x3_supported(q, k, v, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past))
     return ikv::attn_bf16x3(q, k, v, pg, out, n_head, n_head_kv, head_dim, n_q, n_kv, n_past, scale, s);
   const int nq = static_cast<int>(n_q), nk = static_cast<int>(n_kv), np = static_cast<int>(n_past);

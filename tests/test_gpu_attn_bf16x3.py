@@ -41,6 +41,9 @@ SHAPES = [
     (3001, 0, 12, 4, 64),      # two workgroups on a CU
     (130, 70, 6, 1, 96), (200, 0, 10, 5, 80), (500, 0, 12, 4, 32), (333, 9, 4, 2, 4),
     (100, 0, 3, 3, 12), (1, 99, 10, 5, 80), (200, 0, 12, 4, 128),
+    # many blocks of few keys, in either form; the last before and the first past the switch
+    (140, 0, 64, 64, 64), (200, 0, 128, 128, 32), (150, 0, 40, 40, 128), (95, 0, 128, 128, 64), (96, 0, 128, 128, 64),
+    (288, 0, 96, 12, 128), (289, 0, 96, 12, 128),
 ]
 
 
