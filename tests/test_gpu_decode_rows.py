@@ -13,6 +13,7 @@ import pytest
 import ikv
 import oracle
 from ikv import synth
+from test_gpu_norm_rows import EPS, midpoint_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +116,44 @@ def test_a_new_token_without_a_block_is_dropped_and_reported(dev):
                           v_new=dev_t(vn, dev), status=st)
     assert host(st)[0] == 2
     assert np.array_equal(bits(k), k0.view(np.uint32)) and np.array_equal(bits(v), v0.view(np.uint32))
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 12, 4), (64, 8, 1), (128, 10, 2), (128, 6, 2), (256, 10, 2)])
+@pytest.mark.parametrize("which", ["all", "first", "last", "key"])
+def test_rows_in_doubt_take_the_index_order_sum(dev, D, Hq, Hkv, which):
+    """New q and k rows whose norm scale lies on a float rounding midpoint: all
+    of them, one query row in the first or the last lane group, or the key row.
+    The folded step gives the separate kernels' bits, and the appended key the
+    oracle's."""
+    import torch
+    n_kv, pos = 130, 129
+    seed = 7600 + D + Hq
+    th = oracle.rope_theta_table(1e6, D, 200)
+    sn, cs = (dev_t(t, dev) for t in ikv.rope_sincos_table(th))
+    w_q, w_k = (1 + 0.3 * synth.normal(seed + i, (D,)) for i in range(2))
+    k0, v0 = synth.normal(seed + 2, (n_kv, Hkv, D)), synth.normal(seed + 3, (n_kv, Hkv, D))
+    q, kn, vn = (synth.normal(seed + 4 + i, (h, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    hard = midpoint_rows(D, Hq + Hkv, seed + 8)
+    G = Hq // Hkv
+    if which == "all":
+        q, kn = hard[:Hq].copy(), hard[Hq:].copy()
+    elif which == "first":
+        q[::G] = hard[:Hkv]
+    elif which == "last":
+        q[G - 1::G] = hard[:Hkv]
+    else:
+        kn = hard[Hq:].copy()
+    p = torch.tensor([pos], dtype=torch.int32, device=dev)
+    wq_d, wk_d = dev_t(w_q, dev), dev_t(w_k, dev)
+    k, v = dev_t(k0, dev), dev_t(v0, dev)
+    out = ikv.attn_decode_rope(dev_t(q, dev), dev_t(kn, dev), dev_t(vn, dev), k, v, n_kv, wq_d, wk_d,
+                               float(EPS), p, sn, cs)
+    k2, v2 = dev_t(k0, dev), dev_t(v0, dev)
+    qr = ikv.qk_norm_rope(dev_t(q, dev)[None], wq_d, p, float(EPS), sn, cs)[0]
+    kr = ikv.qk_norm_rope(dev_t(kn, dev)[None], wk_d, p, float(EPS), sn, cs)[0]
+    out2 = ikv.attn_decode(qr, k2, v2, n_kv, k_new=kr, v_new=dev_t(vn, dev))
+    assert np.array_equal(bits(out), bits(out2))
+    assert np.array_equal(bits(k), bits(k2)) and np.array_equal(bits(v), bits(v2))
+    want = oracle.rope_neox(oracle.rms_norm(kn[None].astype(np.float32), w_k.astype(np.float32), float(EPS)),
+                            np.array([pos], np.int32), th)
+    assert np.array_equal(bits(k)[pos], np.ascontiguousarray(want[0], np.float32).view(np.uint32))
