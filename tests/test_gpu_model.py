@@ -132,8 +132,9 @@ def test_gemm_unaligned_output_equals_aligned(dev, n_out, k, m):
 def gemm_plan(n_out, k, m):
     import ctypes
     tile, split = ctypes.c_int(), ctypes.c_int()
-    assert ikv.load_bench().ikv_bench_gemm_plan(n_out, k, m, ctypes.byref(tile),
-                                                ctypes.byref(split)) == 0
+    # (the plan that mul_mat runs)
+    assert ikv.load_bench().ikv_bench_gemm_choice(n_out, k, m, ctypes.byref(tile),
+                                                  ctypes.byref(split)) == 0
     return tile.value, split.value
 
 
