@@ -41,6 +41,8 @@ sys.path[:0] = [str(ROOT / "infer-llm_amd"), str(ROOT / "oracle")]
 METRIC = "decode KV-attn GB/s (% HBM peak) @ctx 4096; TPOT ms Qwen3-0.6B F32"
 HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
+# bf16 MFMA, dense, over the six products of bf16 pieces that make one of floats
+PIECES_MFMA_PEAK_TFLOPS = 2500.0 / 6
 N_HEAD, N_HEAD_KV, D, N_LAYER = 16, 8, 128, 28
 TRAFFIC_FILE = ROOT / "profiles" / "decode_append_ctx4096_traffic.json"
 
@@ -57,6 +59,18 @@ def decode_bytes(ctx, n_head=N_HEAD, n_head_kv=N_HEAD_KV, d=D):
 def prefill_flops(p, n_head=N_HEAD, d=D):
     # unmasked (query, key) pairs x (QK^T + PV) = n_head * P(P+1)/2 * 4d
     return n_head * (p * (p + 1) // 2) * 4 * d
+
+
+def prefill_on_pieces(p, n_head=N_HEAD, n_head_kv=N_HEAD_KV):
+    # the library's rule for prompts without a past: more 16-row blocks than CUs
+    blocks = -(-p * (n_head // n_head_kv) // 16) * n_head_kv
+    return blocks > 256 and p > (288 if blocks > 4 * 256 else 256)
+
+
+def mfma_share(tflops, pieces):
+    """The share of the peak of the matrix pipe that the kernel runs on."""
+    peak = PIECES_MFMA_PEAK_TFLOPS if pieces else FP32_MFMA_PEAK_TFLOPS
+    return {"mfma": "bf16 pieces" if pieces else "f32", "mfma_frac": round(tflops / peak, 4)}
 
 
 def seeded(ikv, config, index, shape):
@@ -245,7 +259,7 @@ def prefill_only(torch, ikv, p, reps):
     nbytes = 2 * p * N_HEAD_KV * D * 4  # read and written once
     tf = prefill_flops(p) / t_pre / 1e12
     return {"prefill": {"P": p, "us": round(t_pre * 1e6, 2), "tflops": round(tf, 2),
-                        "mfma_frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4)},
+                        **mfma_share(tf, prefill_on_pieces(p))},
             "append": {"rows": p, "us": round(t_app * 1e6, 2), "bytes": nbytes,
                        "gbs": round(nbytes / t_app / 1e9, 1),
                        "frac": round(nbytes / t_app / 1e9 / HBM_PEAK_GBS, 4)}}
@@ -305,6 +319,7 @@ def gemm_table(torch, ikv):
     """ikv.mul_mat (the MFMA GEMM from 2048 tokens on) against torch.mm (the
     vendor BLAS) at GEMM_SHAPES: each timed as a HIP graph of several
     launches, best of three alternated rounds, after warming the clocks."""
+    import ctypes
     dev = torch.device("cuda:0")
     warm_clocks(torch)
 
@@ -321,6 +336,9 @@ def gemm_table(torch, ikv):
             blas.append(graph_us(torch, lambda: torch.mm(x, w.t(), out=ref), reps))
         o, b = min(ours), min(blas)
         tf = 2 * n * k * m / o / 1e6
+        code, split = ctypes.c_int(), ctypes.c_int()
+        if ikv.load_bench().ikv_bench_gemm_choice(n, k, m, ctypes.byref(code), ctypes.byref(split)):
+            raise RuntimeError("gemm plan")
         rows[name] = {"n_out": n, "k": k, "tokens": m, "us": round(o, 1), "tflops": round(tf, 1),
                       "mfma_frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
                       "blas_us": round(b, 1), "vs_blas": round(o / b, 3),
@@ -1110,7 +1128,7 @@ def main():
             t = time_prefill(torch, ikv, p, 20 if p < 2048 else 10)
             tf = prefill_flops(p) / t / 1e12
             extra["prefill"][str(p)] = {"us": round(t * 1e6, 2), "tflops": round(tf, 2),
-                                        "mfma_frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4)}
+                                        **mfma_share(tf, prefill_on_pieces(p))}
             log(f"[bench] prefill P={p}: {t * 1e6:.1f} us, {tf:.2f} TFLOP/s")
         extra["prefill_gemm"] = gemm_table(torch, ikv)
 
