@@ -38,11 +38,11 @@
 //     of S are summed apart from the small ones.
 //   * What bounds it: the matrix pipe is busy about half the time; the rest
 //     is the VALU work that does not fit behind the MFMAs, the 48 LDS reads
-//     per tile and the two barriers. Measured (us, F32 kernels -> this one,
-//     graphs of 10 launches): Qwen3-8B heads, 4096 tokens 1000 -> 682 (202
-//     TFLOP/s), 777 behind 3319 467 -> 290; 0.6B heads, 2048 tokens 150 ->
-//     122; 12 heads of 64 over 4, 1500 behind 500 232 -> 68; 12 of 128 over 4,
-//     512 tokens 59 -> 35.
+//     per tile and the two barriers. Measured (us, the
+//     kernels before -> this one, graphs): Qwen3-8B heads, 4096 tokens 999 ->
+//     746, 777 behind 3319 487 -> 338; 0.6B heads, 2048 tokens 164 -> 137; 12
+//     heads of 64 over 4, 1500 behind 500 235 -> 63; 32 of 64 over 8, 900
+//     tokens 134 -> 36; 12 of 128 over 4, 512 tokens 58 -> 32.
 //   * What the pieces do not carry: a wave starts over on F32 where its sums
 //     are not finite, or where a split of V or Q dropped bits (floats below
 //     2^-109; V's are looked at one by one, as a dim of small values has only
@@ -50,7 +50,7 @@
 //     probabilities are split times 2^17. That costs 1-3% (0.6B heads, 2048
 //     tokens 112.7 -> 115.7 us cold); one look at a wave's largest output cost
 //     nothing, and missed a small dim among ordinary ones and small keys
-//     against large queries.
+//     against large queries. 2048 tokens with every wave starting over: 790.
 //   * Tried and not kept: two waves per SIMD with Q's last pieces in LDS (0.6B
 //     2048 125, 8B 4096 824: 256 registers leave no room to schedule in); K
 //     and V two tiles ahead (equal); blocks in pairs of a long and a short one
