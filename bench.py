@@ -340,7 +340,7 @@ def gemm_table(torch, ikv):
         if ikv.load_bench().ikv_bench_gemm_choice(n, k, m, ctypes.byref(code), ctypes.byref(split)):
             raise RuntimeError("gemm plan")
         rows[name] = {"n_out": n, "k": k, "tokens": m, "us": round(o, 1), "tflops": round(tf, 1),
-                      "mfma_frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
+                      **mfma_share(tf, code.value >= 5),
                       "blas_us": round(b, 1), "vs_blas": round(o / b, 3),
                       "bit_equal_blas": bool(torch.equal(out, ref))}
         log(f"[bench] gemm {name}: {o:.1f} us ({tf:.1f} TF/s), torch.mm {b:.1f} us, "

@@ -217,6 +217,8 @@ int64_t ikv_attn_decode_replay_limit(int n_head, int n_head_kv, int head_dim, in
  * src/kernels/cuda/kernel_f32.cu:346). MFMA tiles, F32 or (longer prompts)
  * bf16 with every float split into three exact bf16 pieces; K/V tiles staged
  * in LDS and shared by the n_head/n_head_kv query heads of a KV head.
+ * n_kv may be larger than n_past + n_q (a longer cache): rows behind the
+ * prompt are not read.
  * Replaces compute_flash_attn for n_q > 1. Needs no workspace.
  * The MFMA kernel takes head_dim 128 with n_head/n_head_kv 1, 2, 4 or 8;
  * any other head_dim in [1, 512] and any n_head that n_head_kv divides run
